@@ -487,61 +487,350 @@ __global__ void __launch_bounds__(LZ_WG) __attribute__((amdgpu_waves_per_eu(LM =
     }
 }
 
-// Full reorthogonalisation (small sectors), classical Gram-Schmidt pass over the whole basis: workgroup t
-// computes dd[t][b] = scale_t <V[t][.][b], v_{j+1}[.][b]> for the lanes whose step j has t <= j; workgroups
-// t >= maxit do the same for the lane's frozen vectors Y[t - maxit] (t - maxit < nlock[b]; unit norm), so that
-// a deflation pass stays orthogonal to the eigenvectors the earlier passes froze.
-template <typename XT, int B>
-__global__ void __launch_bounds__(LZ_WG) k_lz_fr_dots(LzArgs<XT> a, double* __restrict__ dd) {
-    __shared__ double lds[LZ_WG / 64 * B];
-    const int t = blockIdx.x;
-    const int b = threadIdx.x % B;
-    const int j = a.st.step[b];
-    const bool frozen = t >= a.maxit;
-    const bool act = a.st.active[b] != 0 && j < a.maxit && (frozen ? t - a.maxit < a.st.nlock[b] : t <= j);
-    double acc = 0.0;
-    if (act) {
-        const XT* vt = frozen ? a.Y + static_cast<int64_t>(t - a.maxit) * a.vs : a.V + static_cast<int64_t>(t) * a.vs;
-        const XT* vn = a.V + static_cast<int64_t>(j + 1) * a.vs;
-        for (int64_t r = threadIdx.x / B; r < a.D; r += LZ_WG / B) acc += to_d(vt[r * B + b]) * to_d(vn[r * B + b]);
-        if (!frozen) acc *= a.st.scale[t * B + b];
-    }
-    lz_block_put<B>(acc, 0, lds, dd, B);
+// ---- full reorthogonalisation (small sectors, FP64) ------------------------------------------------------------
+// After K1 a step is three or four launches instead of K2, two Gram-Schmidt passes and two reductions:
+//   dots    c_t = scale_t <V_t, w> for every stored vector t <= j and <Y_l, w> for the lane's frozen vectors, with
+//           w = H v_j - beta_j v_{j-1} - alpha_j v_j formed on the fly from W, v_j and K1's alpha partials
+//   (sum)   the row chunks' partial dot products added up (batches; narrow engines add them in `update`)
+//   update  v_{j+1} = w - sum_t c_t scale_t V_t - sum_l d_l Y_l, partials of ||v_{j+1}||^2
+//   beta    alpha_j, beta_{j+1}, the step counter
+// One classical Gram-Schmidt pass: w has been made orthogonal to v_j and v_{j-1} by the recurrence, and its
+// components on the other stored vectors are rounding (measured: ||c|| <= 4e-14 ||v_{j+1}||, 2e-11 where the Krylov
+// space of a 126-state sector runs out), so the pass leaves them at the rounding of the pass itself.  A lane
+// whose ||c|| exceeds LZ_FR_AGAIN ||v_{j+1}|| gets its second pass in `beta` (the criterion of Daniel, Gragg, Kaufman
+// and Stewart, Math. Comp. 30, 772-795, 1976; their bound allows ||c|| of the order of ||v||).
+// Bound: the basis is read twice a step (2 (j + 1) D B doubles) out of L2 and the Infinity Cache; the narrow
+// engines are bound by the latency of their four launches.  Work is cut into row chunks whose number depends on
+// D B alone and into single basis vectors, never by another lane's step count, so a lane's sums are the same
+// alone and in a mix.
+constexpr int LZ_FR_WG = 256;
+constexpr int LZ_FR_T = 4;              // basis vectors per workgroup pass of the dots (w is read once for all four)
+constexpr int LZ_FR_CHUNKS = 64;        // row chunks at most
+constexpr int LZ_FR_CHUNK = 1024;       // elements (rows x lanes) of a chunk at least: four loads of each vector per thread
+constexpr int LZ_FR_GRID = 1024;        // workgroups of the dots: four per CU
+constexpr int LZ_FR_UPD_GRID = 2048;    // workgroups of the update (rows of norm partials)
+constexpr int LZ_FR_CS = 4096;          // coefficients staged at once (32 KB)
+constexpr double LZ_FR_AGAIN = 1e-2;    // ||c|| / ||v_{j+1}|| above which a lane gets a second pass
+
+struct LzFrSplit {
+    int nR = 1;         // row chunks
+    int64_t per = 512;  // elements per chunk, a multiple of 2 LZ_FR_WG
+    int capv = 0;       // coefficient rows of the Krylov slots (multiple of LZ_FR_T)
+    int rows = 0;       // and of the frozen vectors after them
+};
+
+static LzFrSplit lz_fr_split(int64_t vs, int cap, int ymax) {
+    LzFrSplit f;
+    const int64_t n = std::min<int64_t>(std::max<int64_t>((vs + LZ_FR_CHUNK - 1) / LZ_FR_CHUNK, 1), LZ_FR_CHUNKS);
+    const int64_t q = 2 * LZ_FR_WG;
+    f.per = ((vs + n - 1) / n + q - 1) / q * q;
+    f.nR = static_cast<int>((vs + f.per - 1) / f.per);
+    f.capv = (cap + LZ_FR_T - 1) / LZ_FR_T * LZ_FR_T;
+    f.rows = f.capv + (ymax + LZ_FR_T - 1) / LZ_FR_T * LZ_FR_T;
+    return f;
 }
 
-// v_{j+1} -= sum_{t <= j} dd[t] scale_t V[t] + sum_{l < nlock} dd[maxit + l] Y[l]; the last pass also refreshes
-// the current vector and writes the partials of ||v_{j+1}||^2 (as K2 does)
-template <typename XT, int B>
-__global__ void __launch_bounds__(LZ_WG) k_lz_fr_axpy(LzArgs<XT> a, const double* __restrict__ dd, int last) {
-    __shared__ double lds[LZ_WG / 64 * B];
-    const int b = threadIdx.x % B;
-    const int j = a.st.step[b];
-    const int nfz = a.st.nlock[b];
+// largest step of the iterating lanes (-1: none) and their largest frozen set; every thread gets them (each wave
+// holds all B <= 64 lanes)
+template <int B>
+__device__ __forceinline__ void lz_fr_extent(int j, int nl, bool act, int& jm, int& nz) {
+    jm = act ? j : -1;
+    nz = act ? nl : 0;
+#pragma unroll
+    for (int o = 1; o < B; o <<= 1) {
+        jm = max(jm, __shfl_xor(jm, o, 64));
+        nz = max(nz, __shfl_xor(nz, o, 64));
+    }
+}
+
+// nk1 > 0: alpha_j is the sum of K1's nk1 partial rows, formed by every workgroup (the same sum in the same order);
+// workgroup 0 records it.  nk1 = 0: st.sums holds it already.
+template <int B>
+__global__ void __launch_bounds__(LZ_FR_WG) k_lz_fr_dots(LzArgs<double> a, LzFrSplit f, int nk1, double* __restrict__ pd) {
+    constexpr int NWAVE = LZ_FR_WG / 64;
+    __shared__ double red[NWAVE][LZ_FR_T][B];
+    __shared__ double als[B];
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, b = threadIdx.x % B;
+    const int j = a.st.step[b], nl = a.st.nlock[b];
     const bool act = a.st.active[b] != 0 && j < a.maxit;
-    constexpr int ROWS = LZ_WG / B;
-    const int64_t ntile = (a.D + ROWS - 1) / ROWS;
-    const int64_t per = (ntile + gridDim.x - 1) / gridDim.x;
-    const int64_t t0 = min(static_cast<int64_t>(blockIdx.x) * per, ntile), t1 = min(t0 + per, ntile);
-    double pn = 0.0;
-    if (act) {
-        XT* vn = a.V + static_cast<int64_t>(j + 1) * a.vs;
-        for (int64_t tt = t0; tt < t1; ++tt) {
-            const int64_t r = tt * ROWS + threadIdx.x / B;
-            if (r >= a.D) continue;
-            const int64_t idx = r * B + b;
-            double w = to_d(vn[idx]);
-            for (int t = 0; t <= j; ++t) w -= dd[t * B + b] * a.st.scale[t * B + b] * to_d(a.V[static_cast<int64_t>(t) * a.vs + idx]);
-            for (int l = 0; l < nfz; ++l) w -= dd[(a.maxit + l) * B + b] * to_d(a.Y[static_cast<int64_t>(l) * a.vs + idx]);
-            const XT wr = static_cast<XT>(w);
-            vn[idx] = wr;
-            if (last) {
-                a.Xc[idx] = wr;
-                const double wd = to_d(wr);
-                pn += wd * wd;
+    int jm, nz;
+    lz_fr_extent<B>(j, nl, act, jm, nz);
+    if (jm < 0) return;  // uniform
+    if (nk1 > 0) {
+        double s = 0.0;
+        for (int w = threadIdx.x / B; w < nk1; w += LZ_FR_WG / B) s += a.st.part[static_cast<size_t>(w) * B + b];
+#pragma unroll
+        for (int o = B; o < 64; o <<= 1) s += __shfl_xor(s, o, 64);
+        if (lane < B) red[wid][0][lane] = s;
+        __syncthreads();
+        if (threadIdx.x < B) {
+            double t = 0.0;
+            for (int w = 0; w < NWAVE; ++w) t += red[w][0][threadIdx.x];
+            als[threadIdx.x] = t;
+            if (blockIdx.x == 0) a.st.sums[threadIdx.x] = t;
+        }
+    } else if (threadIdx.x < B) {
+        als[threadIdx.x] = a.st.sums[threadIdx.x];
+    }
+    __syncthreads();
+    const double coef = act ? (als[b] - lz_sigma<B>(a.st, b, j)) * a.st.scale[j * B + b] : 0.0;
+    const int nTv = jm / LZ_FR_T + 1, nT = nTv + (nz + LZ_FR_T - 1) / LZ_FR_T;
+    const int cr = blockIdx.x % f.nR;
+    const int64_t e0 = static_cast<int64_t>(cr) * f.per + threadIdx.x;
+    const int64_t e1 = min(static_cast<int64_t>(cr + 1) * f.per, a.vs);
+    for (int ct = blockIdx.x / f.nR; ct < nT; ct += gridDim.x / f.nR) {
+        const bool fz = ct >= nTv;
+        const int t0 = (fz ? ct - nTv : ct) * LZ_FR_T, last = fz ? nz - 1 : jm;
+        const double* p[LZ_FR_T];
+        double acc[LZ_FR_T];
+#pragma unroll
+        for (int q = 0; q < LZ_FR_T; ++q) {
+            p[q] = (fz ? a.Y : a.V) + static_cast<int64_t>(min(t0 + q, last)) * a.vs;
+            acc[q] = 0.0;
+        }
+        int64_t e = e0;
+        // two elements of w and of the four vectors in flight per thread; a slot a lane has not reached yet adds to
+        // that (slot, lane) only, which is dropped below
+        for (; e + LZ_FR_WG < e1; e += 2 * LZ_FR_WG) {
+            const double w0 = a.W[e], x0 = a.Xc[e], w1 = a.W[e + LZ_FR_WG], x1 = a.Xc[e + LZ_FR_WG];
+            double v0[LZ_FR_T], v1[LZ_FR_T];
+#pragma unroll
+            for (int q = 0; q < LZ_FR_T; ++q) {
+                v0[q] = p[q][e];
+                v1[q] = p[q][e + LZ_FR_WG];
+            }
+            const double y0 = w0 - coef * x0, y1 = w1 - coef * x1;
+#pragma unroll
+            for (int q = 0; q < LZ_FR_T; ++q) {
+                acc[q] += v0[q] * y0;
+                acc[q] += v1[q] * y1;
             }
         }
+        if (e < e1) {
+            const double y0 = a.W[e] - coef * a.Xc[e];
+#pragma unroll
+            for (int q = 0; q < LZ_FR_T; ++q) acc[q] += p[q][e] * y0;
+        }
+#pragma unroll
+        for (int q = 0; q < LZ_FR_T; ++q) {
+            double t = acc[q];
+#pragma unroll
+            for (int o = B; o < 64; o <<= 1) t += __shfl_xor(t, o, 64);
+            if (lane < B) red[wid][q][lane] = t;
+        }
+        __syncthreads();
+        for (int i = threadIdx.x; i < LZ_FR_T * B; i += LZ_FR_WG) {
+            const int q = i / B, t = t0 + q;  // i % B == b (LZ_FR_WG is a multiple of B)
+            const bool ok = act && (fz ? t < nl : t <= j);
+            double s = 0.0;
+            if (ok) {
+                for (int w = 0; w < NWAVE; ++w) s += red[w][q][b];
+                if (!fz) s *= a.st.scale[t * B + b];
+            }
+            pd[(static_cast<size_t>(cr) * f.rows + (fz ? f.capv + t : t)) * B + b] = s;
+        }
+        __syncthreads();
     }
-    if (last) lz_block_put<B>(pn, 0, lds, a.st.part, B);
+}
+
+// c[row][b] = sum of the row chunks' partial dot products, for the rows the lane uses
+template <int B>
+__global__ void __launch_bounds__(LZ_FR_WG) k_lz_fr_sum(LzArgs<double> a, LzFrSplit f, const double* __restrict__ pd,
+                                                        double* __restrict__ c) {
+    const int i = blockIdx.x * LZ_FR_WG + threadIdx.x;
+    if (i >= f.rows * B) return;
+    const int b = i % B, row = i / B, j = a.st.step[b];
+    if (a.st.active[b] == 0 || j >= a.maxit || !(row < f.capv ? row <= j : row - f.capv < a.st.nlock[b])) return;
+    double s = 0.0;
+#pragma unroll 8
+    for (int r = 0; r < f.nR; ++r) s += pd[static_cast<size_t>(r) * f.rows * B + i];
+    c[i] = s;
+}
+
+// A tile is 64 EPT elements.  The NG waves of a workgroup take the basis vectors t = wave (mod NG), so that a
+// thread has a short chain of loads even where D B leaves few threads (D = 6,435, one lane: 101 workgroups of
+// sixteen waves, six or seven vectors each at step 100), and their partial sums meet in LDS.  nparts > 0: the
+// coefficients are the sums of that many chunk partials at `c` (narrow engines), else c holds them.
+template <int B, int NG, int EPT>
+__global__ void __launch_bounds__(64 * NG) k_lz_fr_update(LzArgs<double> a, LzFrSplit f, const double* __restrict__ c, int nparts,
+                                                          double* __restrict__ csq) {
+    constexpr int WG = 64 * NG, TE = 64 * EPT, TB = LZ_FR_CS / B;
+    __shared__ double cs[LZ_FR_CS];
+    __shared__ double red[NG][TE];
+    const int g = threadIdx.x >> 6, ln = threadIdx.x & 63, b = threadIdx.x % B;
+    const int j = a.st.step[b], nl = a.st.nlock[b];
+    const bool act = a.st.active[b] != 0 && j < a.maxit;
+    int jm, nz;
+    lz_fr_extent<B>(j, nl, act, jm, nz);
+    if (jm < 0) return;  // uniform
+    const double coef = act ? (a.st.sums[b] - lz_sigma<B>(a.st, b, j)) * a.st.scale[j * B + b] : 0.0;
+    double* vn = a.V + static_cast<int64_t>(j + 1) * a.vs;
+    double pn = 0.0, sq = 0.0;
+    const int64_t ntile = (a.vs + TE - 1) / TE;
+    for (int64_t tile = blockIdx.x; tile < ntile; tile += gridDim.x) {
+        // this thread's own element of the tile (waves 0 .. EPT - 1) and the columns it sums (every wave)
+        const int64_t own = tile * TE + threadIdx.x;
+        const bool mine = threadIdx.x < TE && own < a.vs && act;
+        const double w0 = mine ? a.W[own] : 0.0, x0 = mine ? a.Xc[own] : 0.0;
+        int64_t e[EPT];
+        double acc[EPT];
+#pragma unroll
+        for (int u = 0; u < EPT; ++u) {
+            e[u] = min(tile * TE + u * 64 + ln, a.vs - B + b);  // a valid element of the same lane past the end
+            acc[u] = 0.0;
+        }
+        for (int fz = 0; fz < 2; ++fz) {
+            const int n = fz ? nz : jm + 1;                          // uniform
+            const int mineN = act ? (fz ? nl : j + 1) : 0;           // this lane's
+            const double* base = fz ? a.Y : a.V;
+            const int row0 = fz ? f.capv : 0;
+            for (int t0 = 0; t0 < n; t0 += TB) {
+                const int t1 = min(t0 + TB, n);
+                __syncthreads();
+                for (int i = threadIdx.x; i < (t1 - t0) * B; i += WG) {
+                    const int t = t0 + i / B;
+                    double s = 0.0;
+                    if (t < mineN) {  // i % B == b
+                        const size_t at = static_cast<size_t>(row0 + t) * B + b;
+                        if (nparts > 0) {
+                            for (int r = 0; r < nparts; ++r) s += c[static_cast<size_t>(r) * f.rows * B + at];
+                        } else {
+                            s = c[at];
+                        }
+                        if (tile == 0) sq += s * s;
+                        if (!fz) s *= a.st.scale[t * B + b];
+                    }
+                    cs[i] = s;
+                }
+                __syncthreads();
+                const int te = min(t1, mineN);
+                for (int t = t0 + g; t < te; t += 4 * NG) {
+                    double v[4][EPT], cc[4];
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        // past the lane's last vector: that vector again, with a zero coefficient
+                        const int tq = min(t + q * NG, te - 1);
+                        cc[q] = t + q * NG < te ? cs[(tq - t0) * B + b] : 0.0;
+#pragma unroll
+                        for (int u = 0; u < EPT; ++u) v[q][u] = base[static_cast<int64_t>(tq) * a.vs + e[u]];
+                    }
+#pragma unroll
+                    for (int q = 0; q < 4; ++q)
+#pragma unroll
+                        for (int u = 0; u < EPT; ++u) acc[u] += cc[q] * v[q][u];
+                }
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < EPT; ++u) red[g][u * 64 + ln] = acc[u];
+        __syncthreads();
+        if (mine) {
+            double s = 0.0;
+#pragma unroll
+            for (int q = 0; q < NG; ++q) s += red[q][threadIdx.x];
+            const double v = (w0 - coef * x0) - s;
+            vn[own] = v;
+            a.Xc[own] = v;
+            pn += v * v;
+        }
+        __syncthreads();
+    }
+    // norm partials (waves 0 .. EPT - 1 hold them), and ||c||^2 per lane from workgroup 0 (tile 0)
+#pragma unroll
+    for (int o = B; o < 64; o <<= 1) pn += __shfl_xor(pn, o, 64);
+    if (ln < B && g < EPT) red[g][ln] = pn;
+    __syncthreads();
+    if (threadIdx.x < B) {
+        double s = 0.0;
+#pragma unroll
+        for (int q = 0; q < EPT; ++q) s += red[q][threadIdx.x];
+        a.st.part[static_cast<size_t>(blockIdx.x) * B + threadIdx.x] = s;
+    }
+    if (blockIdx.x == 0) {  // uniform over the workgroup
+        __syncthreads();
+#pragma unroll
+        for (int o = B; o < 64; o <<= 1) sq += __shfl_xor(sq, o, 64);
+        if (ln < B) red[g][ln] = sq;
+        __syncthreads();
+        if (threadIdx.x < B) {
+            double s = 0.0;
+            for (int q = 0; q < NG; ++q) s += red[q][threadIdx.x];
+            csq[threadIdx.x] = s;
+        }
+    }
+}
+
+// One workgroup: ||v_{j+1}||^2 from the update's partials, the second pass of the lanes that need one (c: scratch for
+// their coefficients), then alpha_j, beta_{j+1}, 1 / beta and the step of every iterating lane.  A lane whose
+// beta is at the level at which the analysis cuts T (1e-12 of its coefficients) is left as it is.
+template <int B>
+__global__ void __launch_bounds__(LZ_RED_WG) k_lz_fr_beta(LzArgs<double> a, LzFrSplit f, int nwg, const double* __restrict__ csq,
+                                                          double* c) {
+    constexpr int NWAVE = LZ_RED_WG / 64;
+    __shared__ double red[NWAVE][B];
+    __shared__ double n2[B];
+    __shared__ int again[B];
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, b = threadIdx.x % B;
+    double s = 0.0;
+    for (int w = threadIdx.x / B; w < nwg; w += LZ_RED_WG / B) s += a.st.part[static_cast<size_t>(w) * B + b];
+#pragma unroll
+    for (int o = B; o < 64; o <<= 1) s += __shfl_xor(s, o, 64);
+    if (lane < B) red[wid][lane] = s;
+    __syncthreads();
+    const int j = a.st.step[b];
+    const bool act = a.st.active[b] != 0 && j < a.maxit;
+    const double al = a.st.sums[b];
+    if (threadIdx.x < B) {
+        double t = 0.0;
+        for (int w = 0; w < NWAVE; ++w) t += red[w][threadIdx.x];
+        n2[threadIdx.x] = t;
+        const double cut = 1e-12 * (fabs(al) + (j > 0 ? a.st.beta[j * B + b] : 0.0));
+        again[threadIdx.x] = act && csq[b] > LZ_FR_AGAIN * LZ_FR_AGAIN * t && t > cut * cut;
+    }
+    __syncthreads();
+    for (int l = 0; l < B; ++l) {
+        if (!again[l]) continue;  // uniform
+        const int jl = a.st.step[l], nv = jl + 1, nq = nv + a.st.nlock[l];
+        double* vn = a.V + static_cast<int64_t>(jl + 1) * a.vs;
+        for (int q = wid; q < nq; q += NWAVE) {
+            const double* v = q < nv ? a.V + static_cast<int64_t>(q) * a.vs : a.Y + static_cast<int64_t>(q - nv) * a.vs;
+            double t = 0.0;
+            for (int64_t r = lane; r < a.D; r += 64) t += v[r * B + l] * vn[r * B + l];
+#pragma unroll
+            for (int o = 32; o >= 1; o >>= 1) t += __shfl_xor(t, o, 64);
+            if (lane == 0) {
+                const double sc = q < nv ? a.st.scale[q * B + l] : 1.0;
+                c[q] = t * sc * sc;  // the coefficient of the stored (unnormalised) vector
+            }
+        }
+        __syncthreads();
+        double pn = 0.0;
+        for (int64_t r = threadIdx.x; r < a.D; r += LZ_RED_WG) {
+            double w = vn[r * B + l];
+            for (int q = 0; q < nq; ++q)
+                w -= c[q] * (q < nv ? a.V[static_cast<int64_t>(q) * a.vs + r * B + l] : a.Y[static_cast<int64_t>(q - nv) * a.vs + r * B + l]);
+            vn[r * B + l] = w;
+            a.Xc[r * B + l] = w;
+            pn += w * w;
+        }
+#pragma unroll
+        for (int o = 32; o >= 1; o >>= 1) pn += __shfl_xor(pn, o, 64);
+        if (lane == 0) red[wid][0] = pn;
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            double t = 0.0;
+            for (int w = 0; w < NWAVE; ++w) t += red[w][0];
+            n2[l] = t;
+        }
+        __syncthreads();
+    }
+    if (threadIdx.x < B && act) {
+        const double nrm = std::sqrt(n2[b]);
+        a.st.alpha[j * B + b] = al;
+        a.st.beta[(j + 1) * B + b] = nrm;
+        a.st.scale[(j + 1) * B + b] = nrm > 0.0 ? 1.0 / nrm : 0.0;
+        a.st.step[b] = j + 1;
+    }
 }
 
 // V[0][r][b] = r0[r] in storage precision (start vector shared by all b)
@@ -1332,7 +1621,11 @@ class LzEngine final : public LzEngineBase {
         BH_TRY(dalloc(ctx, dnj, B));
         BH_TRY(dalloc(ctx, lock_map, static_cast<size_t>(std::max(LZ_CMAX, ymax)) * B));
         BH_TRY(dalloc(ctx, dno, B));
-        if (fullre) BH_TRY(dalloc(ctx, dd, static_cast<size_t>(slots + ymax) * B));
+        if (fullre) {
+            frs = lz_fr_split(vs, cap, ymax);
+            // the chunks' partial dot products, then the coefficients themselves (also the second pass's scratch)
+            BH_TRY(dalloc(ctx, dd, static_cast<size_t>(frs.nR + 1) * frs.rows * B));
+        }
         st.alpha = st_d.p;
         st.beta = st.alpha + n_alpha;
         st.scale = st.beta + n_beta;
@@ -2571,7 +2864,42 @@ class LzEngine final : public LzEngineBase {
         const int g = std::max(1, std::min((nv + waves - 1) / waves, 64));
         hipLaunchKernelGGL(k_lz_reduce, dim3(g), dim3(LZ_RED_WG), 0, s, part.p, nwg, nv, out);
     }
+    // K1 and the full-reorthogonalisation kernels.  K1's alpha partials are summed by the dots themselves while a
+    // workgroup reads at most 4096 of them (32 KB; 3 us saved a launch), by R1 otherwise.  Chunk partials are
+    // summed by the update while that costs a workgroup at most 32 loads a basis vector (narrow engines), by
+    // k_lz_fr_sum otherwise.
+    void step_fullre() {
+        if constexpr (!MIXED) {
+            launch_k1(0);
+            KTimer kt(ctx, "lanczos_reorth", s);
+            const bool direct = grid_k1 * B <= 4096;
+            if (!direct)
+                hipLaunchKernelGGL((k_lz_reduce_wide<B>), dim3(B), dim3(LZ_RED_WG), 0, s, st, part.p, grid_k1, B, B, 0, st.sums);
+            const int nt = frs.rows / LZ_FR_T;
+            const int gd = frs.nR * std::min(nt, std::max(1, LZ_FR_GRID / frs.nR));
+            hipLaunchKernelGGL((k_lz_fr_dots<B>), dim3(gd), dim3(LZ_FR_WG), 0, s, a, frs, direct ? grid_k1 : 0, dd.p);
+            double* c = dd.p + static_cast<size_t>(frs.nR) * frs.rows * B;
+            const int nparts = frs.nR * B <= 32 ? frs.nR : 0;
+            if (nparts == 0)
+                hipLaunchKernelGGL((k_lz_fr_sum<B>), dim3((frs.rows * B + LZ_FR_WG - 1) / LZ_FR_WG), dim3(LZ_FR_WG), 0, s, a, frs,
+                                   dd.p, c);
+            // sixteen waves a tile of 64 elements while that fills at most four tiles a CU, else four waves and 128
+            const bool narrow = vs <= 65536;
+            const int te = narrow ? 64 : 128;
+            const int gu = static_cast<int>(std::min<int64_t>((vs + te - 1) / te, LZ_FR_UPD_GRID));
+            const double* cin = nparts ? dd.p : c;
+            if (narrow)
+                hipLaunchKernelGGL((k_lz_fr_update<B, 16, 1>), dim3(gu), dim3(1024), 0, s, a, frs, cin, nparts, sums2.p);
+            else
+                hipLaunchKernelGGL((k_lz_fr_update<B, 4, 2>), dim3(gu), dim3(256), 0, s, a, frs, cin, nparts, sums2.p);
+            hipLaunchKernelGGL((k_lz_fr_beta<B>), dim3(1), dim3(LZ_RED_WG), 0, s, a, frs, gu, sums2.p, c);
+        }
+    }
     void step(int LM) {
+        if (fullre) {
+            step_fullre();
+            return;
+        }
         launch_k1(LM);
         {
             KTimer kt(ctx, "lanczos_reduce", s);
@@ -2584,15 +2912,6 @@ class LzEngine final : public LzEngineBase {
             else if (LM == 4) hipLaunchKernelGGL((k_lz_b<XT, B, 4>), dim3(grid_k2), dim3(LZ_WG), 0, s, a);
             else if (LM == 8) hipLaunchKernelGGL((k_lz_b<XT, B, 8>), dim3(grid_k2), dim3(LZ_WG), 0, s, a);
             else hipLaunchKernelGGL((k_lz_b<XT, B, 16>), dim3(grid_k2), dim3(LZ_WG), 0, s, a);
-        }
-        if (fullre) {
-            // two classical Gram-Schmidt passes against every stored Lanczos vector of the lane
-            KTimer kt(ctx, "lanczos_reorth", s);
-            for (int pass = 0; pass < 2; ++pass) {
-                hipLaunchKernelGGL((k_lz_fr_dots<XT, B>), dim3(static_cast<unsigned>(cap + (mult ? ymax : 0))), dim3(LZ_WG), 0,
-                                   s, a, dd.p);
-                hipLaunchKernelGGL((k_lz_fr_axpy<XT, B>), dim3(grid_k2), dim3(LZ_WG), 0, s, a, dd.p, pass);
-            }
         }
         {
             KTimer kt(ctx, "lanczos_reduce", s);
@@ -3005,6 +3324,7 @@ class LzEngine final : public LzEngineBase {
     DevArray<double> W_own, r0_own, st_d, part, sums2, dC, dnorm, dd;
     DevArray<int> st_i, dnj, dno, lock_map;
     size_t n_alpha = 0, n_beta = 0, bytes = 0;
+    LzFrSplit frs;
     LzState st{};
     LzArgs<XT> a{};
     int k1v = 1, grid_rb = 1, grid_rl = 1, grid_k1 = 1, grid_k2 = 1;
@@ -3070,6 +3390,7 @@ size_t bh_engine_bytes(int64_t D, int prec, int B, const bh_lanczos_opts& o) {
     const size_t vs = static_cast<size_t>(D) * Bp;
     const int64_t rpw = std::max<int64_t>(static_cast<int64_t>(LZ_WG / Bp) * LZ_K1_TILES, (D + LZ_K1_GRID_MAX - 1) / LZ_K1_GRID_MAX);
     const int ymax = lz_ymax(D, o);
+    const LzFrSplit frs = lz_fr_split(static_cast<int64_t>(vs), slots - 1, ymax);
     const size_t row_bytes = static_cast<size_t>(std::max(2 * LZ_NVMAX + 1 + 2 * LZ_LMAX, ymax)) * Bp * 8;
     // partial-sum rows: the row-lane and K2 grids, or the staged K1's (up to LZ_PART_BYTES)
     const size_t part_rows = std::max<size_t>(
@@ -3078,7 +3399,7 @@ size_t bh_engine_bytes(int64_t D, int prec, int B, const bh_lanczos_opts& o) {
     return (static_cast<size_t>(slots) + ymax + 1) * vs * es + vs * 8 + static_cast<size_t>(D) * 8 +
            part_rows * row_bytes +
            (static_cast<size_t>(slots) + 2) * Bp * 24 + static_cast<size_t>(3 * LZ_LMAX + 1) * Bp * 8 +
-           (fr ? static_cast<size_t>(slots + ymax) * Bp * 8 : 0);
+           (fr ? static_cast<size_t>(frs.nR + 1) * frs.rows * Bp * 8 : 0);
 }
 
 // Options of the FP64 rerun of a rejected mixed solve: the plain FP64 solver (selective
