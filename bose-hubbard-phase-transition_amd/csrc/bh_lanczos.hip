@@ -58,7 +58,6 @@ constexpr int LZ_K2_GRID = 1024;   // K2 workgroups at most (rows of partial sum
 constexpr int LZ_K1_TILES = 4;         // row groups per K1 workgroup on the row-lane engine
 constexpr int LZ_TUNE_REPS = 3;        // timed launches per K1 variant in the autotuner
 constexpr int LZ_CHECK_MIN = 4;        // fewest steps between two analyses of a lane
-constexpr int64_t LZ_SPEC_MIN_WORK = 4ll << 20;  // D B from which analyses overlap speculative steps
 constexpr int64_t LZ_PART_BYTES = 64ll << 20;  // partial sums of the staged K1 (more workgroups than grid_rl)
 constexpr int LZ_K1_GRID_MAX = 32768;  // K1 workgroups at most (rows of partial sums)
 constexpr int LZ_REFINE_STEPS = 3;         // Davidson steps of the FP64 refinement of a rejected mixed lane
@@ -1491,8 +1490,8 @@ void analyze(const RunHost& rh, int j, double beta_next, int p, Analysis& an) {
     an.theta.assign(p, 0.0);
     an.bound.assign(p, 0.0);
     an.s.assign(p, std::vector<double>(j));
+    bhtri::bisect_lowest(j, a, b, p, lo, hi, an.theta.data());
     for (int i = 0; i < p; ++i) {
-        an.theta[i] = bhtri::bisect(j, a, b, i, lo, hi);
         bhtri::inverse_iteration(j, a, b, an.theta[i], an.tnorm, an.s[i].data());
         an.bound[i] = std::fabs(beta_next * an.s[i][j - 1]);
     }
@@ -2129,18 +2128,16 @@ class LzEngine final : public LzEngineBase {
             for (int b = 0; b < B; ++b)
                 if (act[b] && std::min({nextc[b], cap, jsync[b] + std::max(0, maxsteps - totsync[b])}) <= jsync[b])
                     todo.push_back(b);
-            const int nth = std::max(1, std::min(static_cast<int>(todo.size()),
+            // a thread per two lanes (starting one costs a fraction of an analysis), this one among them
+            const int nth = std::max(1, std::min(static_cast<int>(todo.size() + 1) / 2,
                                                  static_cast<int>(std::thread::hardware_concurrency())));
-            if (nth <= 1) {
-                for (int b : todo) analyse_run(b);
-            } else {
-                std::vector<std::thread> pool;
-                for (int t = 0; t < nth; ++t)
-                    pool.emplace_back([&, t]() {
-                        for (size_t q = t; q < todo.size(); q += nth) analyse_run(todo[q]);
-                    });
-                for (auto& th : pool) th.join();
-            }
+            auto share = [&](int t) {
+                for (size_t q = t; q < todo.size(); q += nth) analyse_run(todo[q]);
+            };
+            std::vector<std::thread> pool;
+            for (int t = 1; t < nth; ++t) pool.emplace_back(share, t);
+            share(0);
+            for (auto& th : pool) th.join();
         }
         bool any_lock = false, any_done = false, any_restart = false, any_deflate = false;
         for (int b = 0; b < B; ++b) {
@@ -2720,11 +2717,10 @@ class LzEngine final : public LzEngineBase {
         e = std::min<int64_t>(e, static_cast<int64_t>(jl[b]) + std::max(0, maxsteps - tot[b]));
         return e;
     }
-    // Speculative steps pay when they keep the device busy for a good part of a host analysis (a few
-    // milliseconds): on for engines of at least LZ_SPEC_MIN_WORK vector elements (D B), whose steps take
-    // hundreds of microseconds; smaller engines analyse at the scheduled steps only.  The rule depends on
-    // the sizes alone, so the sequence of analyses and its results are reproducible.
-    bool speculate() const { return lz_spec_steps() > 0 && vs >= LZ_SPEC_MIN_WORK; }
+    // Speculative steps keep the device busy during a host analysis at every size: an analysis takes 0.1 to 0.4 ms a
+    // lane, eight steps of a small sector 0.2 to 0.7 ms.  A lane that its analysis changes wastes them (three passes
+    // of a D = 6,435 solve: 24 of 345 steps).
+    bool speculate() const { return lz_spec_steps() > 0; }
     // orthogonalisation variant of the next steps: the smallest of 0, 4, 8, 16 locked vectors that covers every
     // iterating lane's current set (a lane's set shrinks back to its frozen vectors at a deflation); none under
     // full reorthogonalisation, whose steps project out the frozen vectors themselves

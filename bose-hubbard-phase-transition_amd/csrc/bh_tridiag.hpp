@@ -47,6 +47,56 @@ inline double bisect(int n, const double* a, const double* b, int idx, double lo
     return 0.5 * (lo + hi);
 }
 
+// the p lowest eigenvalues, each the same sequence of midpoints and counts as bisect(i), eight of them side by side:
+// one Sturm recurrence is a chain of dependent divisions (about 22 cycles a row), eight independent ones keep the
+// divider busy (twelve values of a 150-row T: 0.6 -> 0.1 ms)
+inline void bisect_lowest(int n, const double* a, const double* b, int p, double lo0, double hi0, double* out) {
+    constexpr int W = 8;
+    const double tiny = 1e-300 + 1e-18 * std::fmax(std::fabs(lo0), std::fabs(hi0));
+    std::vector<double> b2(n);
+    for (int t = 1; t < n; ++t) b2[t] = b[t] * b[t];
+    for (int i0 = 0; i0 < p; i0 += W) {
+        const int m = p - i0 < W ? p - i0 : W;
+        double lo[W], hi[W], mid[W], q[W], c[W];
+        bool on[W];
+        for (int i = 0; i < W; ++i) {
+            lo[i] = lo0;
+            hi[i] = hi0;
+            on[i] = i < m;
+        }
+        for (int it = 0; it < 200; ++it) {
+            bool any = false;
+            for (int i = 0; i < W; ++i) {
+                mid[i] = 0.5 * (lo[i] + hi[i]);
+                if (on[i] && (mid[i] <= lo[i] || mid[i] >= hi[i] ||
+                              hi[i] - lo[i] <= 4.0e-16 * std::fmax(std::fabs(lo[i]), std::fabs(hi[i]))))
+                    on[i] = false;
+                any = any || on[i];
+            }
+            if (!any) break;
+            for (int i = 0; i < W; ++i) {
+                const double d = a[0] - mid[i];
+                q[i] = d == 0.0 ? -tiny : d;
+                c[i] = q[i] < 0 ? 1.0 : 0.0;
+            }
+            for (int t = 1; t < n; ++t) {
+                const double at = a[t], bt = b2[t];
+                for (int i = 0; i < W; ++i) {
+                    const double d = (at - mid[i]) - bt / q[i];
+                    q[i] = d == 0.0 ? -tiny : d;
+                    c[i] += q[i] < 0 ? 1.0 : 0.0;
+                }
+            }
+            for (int i = 0; i < W; ++i) {
+                if (!on[i]) continue;
+                if (c[i] > i0 + i) hi[i] = mid[i];
+                else lo[i] = mid[i];
+            }
+        }
+        for (int i = 0; i < m; ++i) out[i0 + i] = 0.5 * (lo[i] + hi[i]);
+    }
+}
+
 // inverse iteration: unit eigenvector s of T for the eigenvalue approximation theta
 inline void inverse_iteration(int n, const double* a, const double* b, double theta, double tnorm, double* s) {
     std::vector<double> dl(n), d(n), du(n), du2(n), x(n);
