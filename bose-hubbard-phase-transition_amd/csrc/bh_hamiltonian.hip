@@ -184,20 +184,6 @@ __global__ void __launch_bounds__(256) k_spdm_sum(const double* __restrict__ par
     if (threadIdx.x == 0) out[blockIdx.x] = (red[0] + red[1]) + (red[2] + red[3]);
 }
 
-__global__ void k_ham_expand64(int64_t nnz, const uint32_t* __restrict__ words, int cb, const double* __restrict__ table,
-                               int32_t* __restrict__ col, double* __restrict__ val) {
-    const int64_t k = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (k >= nnz) return;
-    const uint32_t w = words[k];
-    col[k] = static_cast<int32_t>(w >> cb);
-    val[k] = -table[w & ((1u << cb) - 1u)];
-}
-
-__global__ void k_f32_to_f64(int64_t n, const float* __restrict__ a, double* __restrict__ b) {
-    const int64_t k = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (k < n) b[k] = static_cast<double>(a[k]);
-}
-
 // out[0]: longest row; out[1]: largest row sum of |T| (FP32 bits, non-negative); out[2], out[3]: min, max of V
 __global__ void k_row_stats(int64_t D, const int32_t* __restrict__ row_ptr, const uint32_t* __restrict__ words, int cb,
                             const double* __restrict__ table, const float* __restrict__ diag, int* __restrict__ out) {
@@ -321,38 +307,18 @@ static int free_ham(bh_ham* h) {
     for (auto& kv : h->rowblocks) bh_dev_free(ctx, kv.second.first, static_cast<size_t>(kv.second.second + 1) * 8);
     const size_t tab = (static_cast<size_t>(1) << h->code_bits);
     bh_dev_free(ctx, h->row_ptr, static_cast<size_t>(h->D + 1) * sizeof(int32_t));
-    bh_dev_free(ctx, h->words, static_cast<size_t>(h->nnz ? h->nnz : 1) * sizeof(uint32_t));
+    bh_dev_free(ctx, h->words, static_cast<size_t>(h->nnz + BH_WORDS_PAD) * sizeof(uint32_t));
     bh_dev_free(ctx, h->diag, static_cast<size_t>(h->D) * sizeof(float));
     bh_dev_free(ctx, h->table, tab * sizeof(double));
     bh_dev_free(ctx, h->table32, tab * sizeof(float));
-    bh_dev_free(ctx, h->col64, static_cast<size_t>(h->nnz ? h->nnz : 1) * sizeof(int32_t));
-    bh_dev_free(ctx, h->val64, static_cast<size_t>(h->nnz ? h->nnz : 1) * sizeof(double));
-    bh_dev_free(ctx, h->diag64, static_cast<size_t>(h->D) * sizeof(double));
     bh_dev_free(ctx, h->lex_of_pos, static_cast<size_t>(h->D) * sizeof(int32_t));
     delete h;
     return BH_OK;
 }
 
+// Both precisions read the packed words, so there is nothing to build; the call is what bh_spmv_noalloc asks for.
 int bh_ham_prepare_locked(bh_ham* h, int prec) {
-    bh_ctx* ctx = h->ctx;
-    if (prec != BH_PREC_FP64 || h->col64) return BH_OK;
-    const size_t nz = static_cast<size_t>(h->nnz ? h->nnz : 1);
-    DevArray<int32_t> c;
-    DevArray<double> v, d;
-    BH_TRY(c.alloc(ctx, nz));
-    BH_TRY(v.alloc(ctx, nz));
-    BH_TRY(d.alloc(ctx, static_cast<size_t>(h->D)));
-    hipStream_t s = ctx->stream;
-    if (h->nnz)
-        hipLaunchKernelGGL(k_ham_expand64, dim3(static_cast<unsigned>((h->nnz + 255) / 256)), dim3(256), 0, s, h->nnz,
-                           h->words, h->code_bits, h->table, c.p, v.p);
-    hipLaunchKernelGGL(k_f32_to_f64, dim3(static_cast<unsigned>((h->D + 255) / 256)), dim3(256), 0, s, h->D, h->diag, d.p);
-    BH_HIP(ctx, hipGetLastError());
-    BH_HIP(ctx, hipStreamSynchronize(s));
-    h->col64 = c.release();
-    h->val64 = v.release();
-    h->diag64 = d.release();
-    h->bytes64 = nz * (sizeof(int32_t) + sizeof(double)) + static_cast<size_t>(h->D) * sizeof(double);
+    if (prec == BH_PREC_FP64) h->prepared64 = true;
     return BH_OK;
 }
 
@@ -460,7 +426,7 @@ int bh_hamiltonian_build(bh_ctx* ctx, const bh_basis* b, const int* nbr_off, con
     int64_t nnz = 0;
     BH_TRY(bh_exclusive_scan_i32(ctx, rownnz.p, D, row_ptr.p, &nnz, s));
     rownnz.reset();
-    BH_TRY(words.alloc(ctx, static_cast<size_t>(nnz ? nnz : 1)));
+    BH_TRY(words.alloc(ctx, static_cast<size_t>(nnz + BH_WORDS_PAD)));
     const size_t lds_bytes = (static_cast<size_t>(gsize) + static_cast<size_t>(HB_BLOCK) * (E + 1)) * sizeof(uint32_t);
     if (lds_bytes > 64 * 1024) return bh_set_error(ctx, BH_ERANGE, "hamiltonian: rank table too large for LDS");
     {
@@ -521,7 +487,7 @@ int bh_ham_destroy(bh_ham* h) {
 
 int64_t bh_ham_dim(const bh_ham* h) { return h ? h->D : -1; }
 int64_t bh_ham_nnz(const bh_ham* h) { return h ? h->nnz : -1; }
-int64_t bh_ham_device_bytes(const bh_ham* h) { return h ? static_cast<int64_t>(h->bytes + h->bytes64 + h->bytes_rb) : -1; }
+int64_t bh_ham_device_bytes(const bh_ham* h) { return h ? static_cast<int64_t>(h->bytes + h->bytes_rb) : -1; }
 
 int bh_ham_prepare(bh_ham* h, int prec) {
     if (!h) return BH_EINVAL;

@@ -156,15 +156,12 @@ struct bh_ham {
     unsigned flags = 0;
     int max_row = 0;              // longest row
     int32_t* row_ptr = nullptr;   // [D+1]
-    uint32_t* words = nullptr;    // [nnz] column << code_bits | code
+    uint32_t* words = nullptr;    // [nnz + BH_WORDS_PAD] column << code_bits | code
     float* diag = nullptr;        // [D] V (exact small integers)
     double* table = nullptr;      // [1 << code_bits] sqrt(code), exact FP64
     float* table32 = nullptr;     // [1 << code_bits] sqrt(code) rounded to FP32
-    // FP64 CSR (BH_PREC_FP64), materialised on demand
-    int32_t* col64 = nullptr;     // [nnz]
-    double* val64 = nullptr;      // [nnz] -sqrt(code)
-    double* diag64 = nullptr;     // [D]
-    size_t bytes = 0, bytes64 = 0;
+    bool prepared64 = false;      // bh_ham_prepare or bh_spmv has been called for FP64 (bh_spmv_noalloc asks for it)
+    size_t bytes = 0;
     // spectral bounds: V in [vmin, vmax]; the largest row sum of |T| (Gershgorin radius of T)
     double vmin = 0.0, vmax = 0.0, tmax = 0.0;
     std::vector<double> vlevels;  // distinct values of V ascending (host, filled on first use)
@@ -192,6 +189,7 @@ int bh_engine_env();  // BHX_ENGINE (-1 when unset)
 // ---- primes and packed occupation states ------------------------------------------------------------
 
 constexpr int BH_MAX_SITES = 32;
+constexpr int BH_WORDS_PAD = 4;  // words past the last entry that a 16-byte load may read (their values are not used)
 constexpr int BH_STAGE_PRODUCTS_HOST = 2048;  // must equal BH_STAGE_PRODUCTS of the row-block engine
 extern const int bh_primes[BH_MAX_SITES];
 

@@ -7,9 +7,6 @@
 
 #include "bh_internal.hpp"
 
-constexpr int BH_FMT_PACKED = 0;  // 32-bit word: column << code_bits | code, value -sqrt(code)
-constexpr int BH_FMT_CSR64 = 1;   // int32 column + FP64 value
-
 constexpr int BH_WG = 256;  // workgroup size of the operator kernels (4 waves)
 
 template <typename XT>
@@ -17,27 +14,20 @@ __device__ __forceinline__ double to_d(XT v) {
     return static_cast<double>(v);
 }
 
-// Partial sum of one lane over its strided part of row r: sum_k value_k * x[col_k * B + b].
-// For the packed format the table holds +sqrt(code); the caller negates.
-template <typename XT, int B, int G, int FMT>
+// Partial sum of one lane over its strided part of row r: sum_k |value_k| * x[col_k * B + b].
+// The table holds +sqrt(code); the caller negates.
+template <typename XT, int B, int G>
 __device__ __forceinline__ double bh_row_partial(int32_t rs, int32_t re, int g, int b, const uint32_t* __restrict__ words,
-                                                 const int32_t* __restrict__ col64, const double* __restrict__ val64,
                                                  const double* __restrict__ tab, int cb, const XT* __restrict__ x) {
     // two entries per iteration, both loaded unconditionally (the second repeats the row's last entry past the
     // end and adds a zero), in the order of k
     double acc = 0.0;
     for (int32_t k = rs + g; k < re; k += 2 * G) {
         const int32_t k1 = min(k + G, re - 1);
-        double p0, p1;
-        if constexpr (FMT == BH_FMT_PACKED) {
-            const uint32_t mask = (1u << cb) - 1u;
-            const uint32_t w0 = words[k], w1 = words[k1];
-            p0 = tab[w0 & mask] * to_d(x[static_cast<int64_t>(w0 >> cb) * B + b]);
-            p1 = tab[w1 & mask] * to_d(x[static_cast<int64_t>(w1 >> cb) * B + b]);
-        } else {
-            p0 = val64[k] * to_d(x[static_cast<int64_t>(col64[k]) * B + b]);
-            p1 = val64[k1] * to_d(x[static_cast<int64_t>(col64[k1]) * B + b]);
-        }
+        const uint32_t mask = (1u << cb) - 1u;
+        const uint32_t w0 = words[k], w1 = words[k1];
+        const double p0 = tab[w0 & mask] * to_d(x[static_cast<int64_t>(w0 >> cb) * B + b]);
+        const double p1 = tab[w1 & mask] * to_d(x[static_cast<int64_t>(w1 >> cb) * B + b]);
         acc += p0;
         acc += k + G < re ? p1 : 0.0;
     }
@@ -117,10 +107,9 @@ __device__ __forceinline__ int64_t bh_xcd_tile(int64_t wg, int64_t nwg) {
 // interface of the row-lane engine).  rb[] holds (first row, first entry) of every block, then (D, nnz).
 constexpr int BH_STAGE_PRODUCTS = 2048;  // FP64 products per block (16 KB of LDS)
 
-template <typename XT, int B, int FMT, int WG, typename Epi>
+template <typename XT, int B, int WG, typename Epi>
 __device__ __forceinline__ void bh_rowblock_run(int64_t t0, int64_t t1, const int32_t* __restrict__ rb,
                                                 const int32_t* __restrict__ rp, const uint32_t* __restrict__ words,
-                                                const int32_t* __restrict__ col64, const double* __restrict__ val64,
                                                 const double* __restrict__ tab, int cb, const XT* __restrict__ x,
                                                 double* prod, Epi& epi) {
     constexpr int CAP = BH_STAGE_PRODUCTS;  // products per block (entries * B)
@@ -140,12 +129,8 @@ __device__ __forceinline__ void bh_rowblock_run(int64_t t0, int64_t t1, const in
                 const int ic = min(static_cast<int>(threadIdx.x) + u * WG, np - 1);
                 const int32_t k = ks + ic / B;
                 const int bb = ic % B;
-                if constexpr (FMT == BH_FMT_PACKED) {
-                    const uint32_t w = words[k];
-                    v[u] = tab[w & mask] * to_d(x[static_cast<int64_t>(w >> cb) * B + bb]);
-                } else {
-                    v[u] = val64[k] * to_d(x[static_cast<int64_t>(col64[k]) * B + bb]);
-                }
+                const uint32_t w = words[k];
+                v[u] = tab[w & mask] * to_d(x[static_cast<int64_t>(w >> cb) * B + bb]);
             }
 #pragma unroll
             for (int u = 0; u < PER; ++u) prod[threadIdx.x + u * WG] = v[u];
@@ -190,10 +175,9 @@ __device__ __forceinline__ BhVec<T, V> bh_vload(const T* p) {
     return *reinterpret_cast<const BhVec<T, V>*>(p);
 }
 
-template <typename XT, int B, int V, int FMT, int WG, int U, typename Epi>
+template <typename XT, int B, int V, int WG, int U, typename Epi>
 __device__ __forceinline__ void bh_rowlane_run(int64_t r0, int64_t r1, const int32_t* __restrict__ rp,
-                                               const uint32_t* __restrict__ words, const int32_t* __restrict__ col64,
-                                               const double* __restrict__ val64, const double* __restrict__ tab, int cb,
+                                               const uint32_t* __restrict__ words, const double* __restrict__ tab, int cb,
                                                const XT* __restrict__ x, Epi& epi) {
     static_assert(B % V == 0, "V divides B");
     constexpr int TPR = B / V;  // threads per row
@@ -214,29 +198,85 @@ __device__ __forceinline__ void bh_rowlane_run(int64_t r0, int64_t r1, const int
             // every word load and gather of the unrolled step is unconditional and all of them are in flight
             // together (a load under a branch is waited for before the next one is issued).  Such an entry
             // adds a zero product (the x it gathers is one the row already uses).
-            if constexpr (FMT == BH_FMT_PACKED) {
 #pragma unroll
-                for (int u = 0; u < U; ++u) w[u] = words[min(k + u, ke - 1)];
+            for (int u = 0; u < U; ++u) w[u] = words[min(k + u, ke - 1)];
 #pragma unroll
-                for (int u = 0; u < U; ++u) xv[u] = bh_vload<V>(x + static_cast<int64_t>(w[u] >> cb) * B + b0);
+            for (int u = 0; u < U; ++u) xv[u] = bh_vload<V>(x + static_cast<int64_t>(w[u] >> cb) * B + b0);
 #pragma unroll
-                for (int u = 0; u < U; ++u) val[u] = k + u < ke ? tab[w[u] & mask] : 0.0;
-            } else {
-#pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    const int32_t kk = min(k + u, ke - 1);
-                    w[u] = static_cast<uint32_t>(col64[kk]);
-                    const double vv = val64[kk];
-                    val[u] = k + u < ke ? vv : 0.0;
-                }
-#pragma unroll
-                for (int u = 0; u < U; ++u) xv[u] = bh_vload<V>(x + static_cast<int64_t>(w[u]) * B + b0);
-            }
+            for (int u = 0; u < U; ++u) val[u] = k + u < ke ? tab[w[u] & mask] : 0.0;
 #pragma unroll
             for (int u = 0; u < U; ++u)
 #pragma unroll
                 for (int v = 0; v < V; ++v) acc[v] += val[u] * to_d(xv[u].v[v]);
         }
         epi(r, b0, acc);
+    }
+}
+
+// ---- row-tile engine (one thread per row, V = B) -------------------------------------------------------------
+// The row-lane engine with a whole row per thread reads 64 different rows' words per load, each from its own cache
+// line.  Here a wave takes a tile of 64 consecutive rows whose words are one contiguous run: it copies them to its
+// part of LDS with 16-byte loads (all of them in flight, no barrier: only the wave itself reads them) and then walks
+// its rows from there, so that the matrix is one coalesced stream and a row's latency is one gather deep.
+// A tile with more words than the part holds goes in several rounds.  The sum of every row runs over its
+// entries in storage order, as on the row-lane engine, with the same bits.  words must be readable up to a multiple of
+// four past the last entry (BH_WORDS_PAD).
+constexpr int BH_TILE_WORDS = 2048;  // words of a wave's LDS part at most (8 KB)
+
+template <typename XT, int V, int WG, int U, typename Epi>
+__device__ __forceinline__ void bh_rowtile_run(int64_t r0, int64_t r1, const int32_t* __restrict__ rp,
+                                               const uint32_t* __restrict__ words, const double* __restrict__ tab, int cb,
+                                               const XT* __restrict__ x, uint32_t* part, int cap, Epi& epi) {
+    const uint32_t mask = (1u << cb) - 1u;
+    const int lane = threadIdx.x & 63;
+    uint32_t* buf = part + (threadIdx.x >> 6) * cap;
+    for (int64_t base = r0 + (threadIdx.x & ~63); base < r1; base += WG) {
+        const int64_t r = base + lane;
+        const int32_t rs = rp[min(r, r1)], re = rp[min(r + 1, r1)];
+        const int32_t k0 = __shfl(rs, 0, 64), k1 = __shfl(re, 63, 64);
+        double acc[V];
+#pragma unroll
+        for (int v = 0; v < V; ++v) acc[v] = 0.0;
+        // rounds of cap - 4 words from a multiple of four
+        for (int32_t c0 = k0; c0 < k1; c0 += cap - 4) {
+            const int32_t ca = c0 & ~3, c1 = min(c0 + cap - 4, k1);
+            for (int i0 = 0; i0 < c1 - ca; i0 += 1024) {
+                uint4 q[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    // past the run's end: its last four words again
+                    const int32_t k = min(ca + i0 + u * 256 + lane * 4, (c1 - 1) & ~3);
+                    q[u] = *reinterpret_cast<const uint4*>(words + k);
+                }
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    const int i = i0 + u * 256 + lane * 4;
+                    if (i < c1 - ca) *reinterpret_cast<uint4*>(buf + i) = q[u];
+                }
+            }
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            const int32_t ks = max(rs, c0) - ca, ke = min(re, c1) - ca;
+            for (int32_t k = ks; k < ke; k += U) {
+                uint32_t w[U];
+                BhVec<XT, V> xv[U];
+                double val[U];
+#pragma unroll
+                for (int u = 0; u < U; ++u) w[u] = buf[min(k + u, ke - 1)];
+#pragma unroll
+                for (int u = 0; u < U; ++u) xv[u] = bh_vload<V>(x + static_cast<int64_t>(w[u] >> cb) * V);
+#pragma unroll
+                for (int u = 0; u < U; ++u) val[u] = k + u < ke ? tab[w[u] & mask] : 0.0;
+#pragma unroll
+                for (int u = 0; u < U; ++u)
+#pragma unroll
+                    for (int v = 0; v < V; ++v) acc[v] += val[u] * to_d(xv[u].v[v]);
+            }
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        }
+        if (r < r1) epi(r, 0, acc);
     }
 }

@@ -55,7 +55,8 @@ constexpr int LZ_WS_A = 5, LZ_WS_B = 6, LZ_WS_C = 7;  // context workspace slots
                                                        // W, locked vectors, start vector, current vectors)
 constexpr int LZ_GRAPH_STEPS = 8;  // Lanczos steps per captured HIP graph
 constexpr int LZ_K2_GRID = 1024;   // K2 workgroups at most (rows of partial sums for R2; 512 and 2048 measured slower)
-constexpr int LZ_K1_TILES = 4;         // row groups per K1 workgroup on the row-lane engine
+constexpr int LZ_K1_TILES = 4;         // row groups per K1 workgroup on the row-lane engine at most
+constexpr int LZ_K1_FILL = 512;        // K1 workgroups below which it takes fewer row groups (two per CU)
 constexpr int LZ_TUNE_REPS = 3;        // timed launches per K1 variant in the autotuner
 constexpr int LZ_CHECK_MIN = 4;        // fewest steps between two analyses of a lane
 constexpr int64_t LZ_PART_BYTES = 64ll << 20;  // partial sums of the staged K1 (more workgroups than grid_rl)
@@ -89,10 +90,7 @@ struct LzArgs {
     int64_t D;
     const int32_t* row_ptr;
     const uint32_t* words;
-    const int32_t* col64;
-    const double* val64;
-    const float* diag32;
-    const double* diag64;
+    const float* diag;
     const double* table;
     int cb;
     XT* V;         // [slots][D][B] Krylov basis; lane b's vector t at V[t][r][b]
@@ -194,7 +192,7 @@ struct K1Shared {
 // K1 epilogue shared by both operator engines: a thread holds the V vectors b0 .. b0 + V - 1 of its rows.
 // w = J_b T x_b + U_b V x_b - beta_j v_{j-1} (x_b = s_j v_j, the stored vector times its scale) is written
 // to W; the thread accumulates <x_b, w> for alpha.
-template <typename XT, int B, int V, int FMT>
+template <typename XT, int B, int V>
 struct K1Epi {
     const LzArgs<XT>& a;
     const K1Shared<B>& ls;
@@ -205,7 +203,7 @@ struct K1Epi {
     double pa[V];
     __device__ __forceinline__ void operator()(int64_t r, int, const double (&acc)[V]) {
         if (!any) return;  // the row-block engine calls every thread
-        const double d = a.diag32 ? static_cast<double>(a.diag32[r]) : a.diag64[r];
+        const double d = static_cast<double>(a.diag[r]);
         const int64_t idx = r * B + b0;
         const BhVec<XT, V> xv = bh_vload<V>(a.Xc + idx);
         BhVec<XT, V> xm;
@@ -219,7 +217,7 @@ struct K1Epi {
 #pragma unroll
         for (int v = 0; v < V; ++v) {
             const int b = b0 + v;
-            const double hx = (FMT == BH_FMT_PACKED) ? -acc[v] : acc[v];
+            const double hx = -acc[v];
             const double xr = to_d(xv.v[v]) * ls.sj[b];
             const double w = ls.jbs[b] * hx + ls.ub[b] * d * xr - ls.bj[b] * to_d(xm.v[v]);
             wv.v[v] = static_cast<XT>(w - ls.sg[b] * xr);
@@ -230,8 +228,8 @@ struct K1Epi {
 };
 
 // fills the LDS lane table (threads < B) and the thread's view of its V lanes; ends with a barrier
-template <typename XT, int B, int V, int FMT>
-__device__ __forceinline__ void k1_setup(const LzArgs<XT>& a, K1Shared<B>& ls, K1Epi<XT, B, V, FMT>& e) {
+template <typename XT, int B, int V>
+__device__ __forceinline__ void k1_setup(const LzArgs<XT>& a, K1Shared<B>& ls, K1Epi<XT, B, V>& e) {
     if (threadIdx.x < B) {
         const int b = threadIdx.x;
         const int j = a.st.step[b];
@@ -261,56 +259,57 @@ __device__ __forceinline__ void k1_setup(const LzArgs<XT>& a, K1Shared<B>& ls, K
 }
 
 // K1 on the LDS-staged row-block engine (B = 1 in the automatic choice)
-template <typename XT, int B, int FMT>
+template <typename XT, int B>
 __global__ void __launch_bounds__(LZ_WG) k_lz_a_rb(LzArgs<XT> a, const int32_t* __restrict__ rb, int64_t nblocks, int nv) {
     extern __shared__ double smem[];
     double* tab = smem;
-    double* prod = smem + (FMT == BH_FMT_PACKED ? (1 << a.cb) : 0);
+    double* prod = smem + (1 << a.cb);
     __shared__ double lds[LZ_WG / 64 * B];
-    if constexpr (FMT == BH_FMT_PACKED) {
-        for (int i = threadIdx.x; i < (1 << a.cb); i += LZ_WG) tab[i] = a.table[i];
-        __syncthreads();
-    }
+    for (int i = threadIdx.x; i < (1 << a.cb); i += LZ_WG) tab[i] = a.table[i];
     __shared__ K1Shared<B> ls;
-    K1Epi<XT, B, 1, FMT> e{a, ls};
+    K1Epi<XT, B, 1> e{a, ls};
     k1_setup(a, ls, e);
     const int64_t per = (nblocks + gridDim.x - 1) / gridDim.x;
     const int64_t L = bh_xcd_tile(blockIdx.x, gridDim.x);
     const int64_t t0 = min(L * per, nblocks), t1 = min(t0 + per, nblocks);
-    bh_rowblock_run<XT, B, FMT, LZ_WG>(t0, t1, rb, a.row_ptr, a.words, a.col64, a.val64, tab, a.cb, a.Xc, prod, e);
+    bh_rowblock_run<XT, B, LZ_WG>(t0, t1, rb, a.row_ptr, a.words, tab, a.cb, a.Xc, prod, e);
     lz_block_put_v<B, 1>(e.pa, 0, lds, a.st.part, nv);
 }
 
-// K1 on the row-lane engine (B / V threads per row, contiguous row ranges per workgroup)
-template <typename XT, int B, int V, int FMT, int U>
-__device__ __forceinline__ void k1_rowlane(const LzArgs<XT>& a, int64_t rows_per_wg, int nv) {
-    extern __shared__ double tab[];
+// K1 on the row-lane engine (B / V threads per row, contiguous row ranges per workgroup); one thread per row (V = B):
+// the row-tile engine, with `cap` words of LDS per wave
+template <typename XT, int B, int V, int U>
+__device__ __forceinline__ void k1_rowlane(const LzArgs<XT>& a, int64_t rows_per_wg, int nv, int cap) {
+    extern __shared__ __align__(16) double tab[];
     __shared__ double lds[LZ_WG / 64 * B];
-    if constexpr (FMT == BH_FMT_PACKED) {
-        for (int i = threadIdx.x; i < (1 << a.cb); i += LZ_WG) tab[i] = a.table[i];
-    }
+    for (int i = threadIdx.x; i < (1 << a.cb); i += LZ_WG) tab[i] = a.table[i];
     __shared__ K1Shared<B> ls;
-    K1Epi<XT, B, V, FMT> e{a, ls};
+    K1Epi<XT, B, V> e{a, ls};
     k1_setup(a, ls, e);
     const int64_t L = bh_xcd_tile(blockIdx.x, gridDim.x);
     const int64_t r0 = min(L * rows_per_wg, a.D), r1 = min(r0 + rows_per_wg, a.D);
-    if (e.any)
-        bh_rowlane_run<XT, B, V, FMT, LZ_WG, U>(r0, r1, a.row_ptr, a.words, a.col64, a.val64, tab, a.cb, a.Xc, e);
+    if (e.any) {
+        if constexpr (B == V)
+            bh_rowtile_run<XT, V, LZ_WG, U>(r0, r1, a.row_ptr, a.words, tab, a.cb, a.Xc,
+                                            reinterpret_cast<uint32_t*>(tab + (1 << a.cb)), cap, e);
+        else
+            bh_rowlane_run<XT, B, V, LZ_WG, U>(r0, r1, a.row_ptr, a.words, tab, a.cb, a.Xc, e);
+    }
     lz_block_put_v<B, V>(e.pa, 0, lds, a.st.part, nv);
 }
 
 // V <= 4, U = 4: at most 80 VGPRs (six waves per SIMD)
-template <typename XT, int B, int V, int FMT>
+template <typename XT, int B, int V>
 __global__ void __launch_bounds__(LZ_WG) __attribute__((amdgpu_waves_per_eu(6))) k_lz_a_rl(LzArgs<XT> a, int64_t rows_per_wg,
-                                                                                            int nv) {
-    k1_rowlane<XT, B, V, FMT, 4>(a, rows_per_wg, nv);
+                                                                                            int nv, int cap) {
+    k1_rowlane<XT, B, V, 4>(a, rows_per_wg, nv, cap);
 }
 
 // wide variants: V = 8 (two 16-byte gathers per entry and thread) or U = 8, 16 entries of a row in flight
 // (long rows at small B)
-template <typename XT, int B, int V, int FMT, int U>
-__global__ void __launch_bounds__(LZ_WG) k_lz_a_rlw(LzArgs<XT> a, int64_t rows_per_wg, int nv) {
-    k1_rowlane<XT, B, V, FMT, U>(a, rows_per_wg, nv);
+template <typename XT, int B, int V, int U>
+__global__ void __launch_bounds__(LZ_WG) k_lz_a_rlw(LzArgs<XT> a, int64_t rows_per_wg, int nv, int cap) {
+    k1_rowlane<XT, B, V, U>(a, rows_per_wg, nv, cap);
 }
 
 // Dot products of an exact orthogonalisation step (so = 1): partials of <y_l, w> and <y_l, s_j v_j> for the
@@ -1515,6 +1514,15 @@ static int lz_slots(int64_t D, const bh_lanczos_opts& o) {
     return static_cast<int>(std::max<int64_t>(cap, 1)) + 1;
 }
 
+// rows of a K1 workgroup on the row-lane engine: passes of LZ_WG V / B rows, up to LZ_K1_TILES of them while that
+// leaves LZ_K1_FILL workgroups (small sectors: D = 6,435 at one lane is 4 workgroups of four passes, 14.7 us, against
+// 13 of one), more when the grid would exceed LZ_K1_GRID_MAX
+static int64_t lz_k1_rows(int64_t D, int B, int V) {
+    const int64_t pass = std::max<int64_t>(static_cast<int64_t>(LZ_WG) * V / B, 1);
+    const int64_t tiles = std::max<int64_t>(1, std::min<int64_t>(LZ_K1_TILES, D / (pass * LZ_K1_FILL)));
+    return std::max<int64_t>(pass * tiles, (D + LZ_K1_GRID_MAX - 1) / LZ_K1_GRID_MAX);
+}
+
 // Sectors up to this dimension run FP64 Lanczos with full reorthogonalisation: their solves are bound by
 // launch latency, not bandwidth, so FP32 storage buys nothing there, and reorthogonalising against the whole
 // basis (j D B words per step) is cheap.
@@ -1533,9 +1541,8 @@ static int lz_ymax(int64_t D, const bh_lanczos_opts& o) {
 template <typename XT, int B>
 class LzEngine final : public LzEngineBase {
     static constexpr bool MIXED = std::is_same<XT, float>::value;
-    // Both precisions read the packed words: the FP64 table gives the exact matrix values (4 bytes per entry
-    // instead of the 12 of an FP64 CSR), and the diagonal V (small integers) is exact in FP32.
-    static constexpr int FMT = BH_FMT_PACKED;
+    // Both precisions read the packed words: the FP64 table gives the exact matrix values in 4 bytes per entry,
+    // and the diagonal V (small integers) is exact in FP32.
 
    public:
     LzEngine(bh_ctx* c, bh_ham* ham, const bh_lanczos_opts& opts, hipStream_t stream, bool use_ctx_ws)
@@ -1596,10 +1603,10 @@ class LzEngine final : public LzEngineBase {
         BH_TRY(dalloc(ctx, st_d, nd));
         BH_TRY(dalloc(ctx, st_i, static_cast<size_t>(3 * B + 2)));
         const int nvmax = std::max({static_cast<int>(n_sums), 2 * LZ_NVMAX * B, ymax * B});
-        // K1 on the row-lane engine: small row tiles (LZ_K1_TILES row groups of LZ_WG / B rows), many
-        // workgroups in flight; its partial sums need a row per workgroup
-        rpw = std::max<int64_t>(static_cast<int64_t>(LZ_WG / B) * LZ_K1_TILES, (D + LZ_K1_GRID_MAX - 1) / LZ_K1_GRID_MAX);
-        grid_rl = static_cast<int>((D + rpw - 1) / rpw);
+        // K1 on the row-lane engine: its partial sums need a row per workgroup (most at V = 1)
+        grid_rl = 1;
+        for (int V = 1; V <= std::min(B, 8); V *= 2)
+            grid_rl = std::max(grid_rl, static_cast<int>((D + lz_k1_rows(D, B, V) - 1) / lz_k1_rows(D, B, V)));
         // K1 on the staged row-block engine: a workgroup per block up to LZ_K1_GRID_MAX workgroups, within
         // LZ_PART_BYTES of partial sums
         staged_ok = static_cast<int64_t>(h->max_row) * B <= BH_STAGE_PRODUCTS_HOST;
@@ -1670,10 +1677,7 @@ class LzEngine final : public LzEngineBase {
         a = LzArgs<XT>{D,
                        h->row_ptr,
                        h->words,
-                       nullptr,
-                       nullptr,
                        h->diag,
-                       nullptr,
                        h->table,
                        h->code_bits,
                        V,
@@ -1683,7 +1687,9 @@ class LzEngine final : public LzEngineBase {
                        Y,
                        cap,
                        st};
-        shm = FMT == BH_FMT_PACKED ? (static_cast<size_t>(1) << h->code_bits) * sizeof(double) : 0;
+        shm = (static_cast<size_t>(1) << h->code_bits) * sizeof(double);
+        // a wave's words on the row-tile engine, with the table and the lane scalars within 64 KB a workgroup
+        tile_cap = std::min(bh_tile_cap(h), static_cast<int>((65536 - 4096 - shm) / (LZ_WG / 64 * sizeof(uint32_t)) / 64 * 64));
         // K1 variant before the tuner has run: staged row blocks, or one thread per (row, b)
         shm_rb = shm + BH_STAGE_PRODUCTS * sizeof(double);
         set_k1(bh_engine_choice(B, h) == 1 && staged_ok ? 0 : 1);
@@ -2275,9 +2281,9 @@ class LzEngine final : public LzEngineBase {
             BH_HIP(ctx, hipMemcpyAsync(dU.p, Ub.data(), B * 8, hipMemcpyHostToDevice, s));
             for (int i = 0; i < nvf; ++i) {
                 KTimer kt(ctx, "lanczos_finish_spmv", s);
-                SpmvArgs<double> sa{D, h->row_ptr, h->words, nullptr, nullptr, h->diag, nullptr, h->table, h->code_bits,
+                SpmvArgs<double> sa{D, h->row_ptr, h->words, h->diag, h->table, h->code_bits,
                                     dJ.p, dU.p, Yfp + static_cast<int64_t>(i) * vs, HYp + static_cast<int64_t>(i) * vs, 1};
-                BH_TRY(bh_apply(ctx, h, &sa, nullptr, BH_FMT_PACKED, B, s));
+                BH_TRY(bh_apply(ctx, h, sa, BH_KEY_FINISH, B, s));
             }
             BH_HIP(ctx, hipGetLastError());
             BH_TRY(rayleigh_ritz(lanes, nvf, nt, Yfp, HYp));
@@ -2533,9 +2539,9 @@ class LzEngine final : public LzEngineBase {
         }
         for (int i = 0; i < np; ++i) {
             KTimer kt(ctx, "lanczos_finish_spmv", s);
-            SpmvArgs<double> sa{D, h->row_ptr, h->words, nullptr, nullptr, h->diag, nullptr, h->table, h->code_bits,
+            SpmvArgs<double> sa{D, h->row_ptr, h->words, h->diag, h->table, h->code_bits,
                                 dJ.p, dU.p, Tp + static_cast<int64_t>(i) * vs, HTp + static_cast<int64_t>(i) * vs, 1};
-            BH_TRY(bh_apply(ctx, h, &sa, nullptr, BH_FMT_PACKED, B, s));
+            BH_TRY(bh_apply(ctx, h, sa, BH_KEY_FINISH, B, s));
         }
         BH_HIP(ctx, hipGetLastError());
         std::vector<int> lr, n2(B, 0);
@@ -2735,27 +2741,24 @@ class LzEngine final : public LzEngineBase {
     // U = 4, 8, 16 entries of a row in flight) = row-lane engine
     static int k1_V(int var) { return var & 15; }
     static int k1_U(int var) { return 4 << (var >> 4); }
-    // rows of a K1 workgroup on the row-lane engine: LZ_K1_TILES passes of LZ_WG V / B rows, more when the
-    // grid would exceed LZ_K1_GRID_MAX
-    int64_t k1_rows(int var) const {
-        return std::max<int64_t>(static_cast<int64_t>(LZ_WG * k1_V(var) / B) * LZ_K1_TILES,
-                                 (D + LZ_K1_GRID_MAX - 1) / LZ_K1_GRID_MAX);
-    }
+    int64_t k1_rows(int var) const { return lz_k1_rows(D, B, k1_V(var)); }
     void set_k1(int var) {
         k1v = var;
         grid_k1 = var == 0 ? grid_rb : static_cast<int>((D + k1_rows(var) - 1) / k1_rows(var));
         rpw_so = (D + grid_k1 - 1) / grid_k1;
     }
+    // LDS of a row-lane variant: the table, and on the row-tile engine (V = B) each wave's words
+    size_t k1_shm(int V) const { return shm + (V == B ? static_cast<size_t>(LZ_WG / 64) * tile_cap * sizeof(uint32_t) : 0); }
     void launch_k1_var(int var, int nv) {
         if (var == 0) {
-            hipLaunchKernelGGL((k_lz_a_rb<XT, B, FMT>), dim3(grid_rb), dim3(LZ_WG), shm_rb, s, a, rblk, nrblk, nv);
+            hipLaunchKernelGGL((k_lz_a_rb<XT, B>), dim3(grid_rb), dim3(LZ_WG), shm_rb, s, a, rblk, nrblk, nv);
             return;
         }
         const int64_t rows = k1_rows(var);
         const dim3 g(static_cast<unsigned>((D + rows - 1) / rows));
 #define K1W(VV, UU)                                                                                    \
     if (var == VV + 16 * (UU == 4 ? 0 : (UU == 8 ? 1 : 2))) {                                          \
-        hipLaunchKernelGGL((k_lz_a_rlw<XT, B, VV, FMT, UU>), g, dim3(LZ_WG), shm, s, a, rows, nv);     \
+        hipLaunchKernelGGL((k_lz_a_rlw<XT, B, VV, UU>), g, dim3(LZ_WG), k1_shm(VV), s, a, rows, nv, tile_cap);  \
         return;                                                                                        \
     }
         if constexpr (B >= 8 && sizeof(XT) == 4) K1W(8, 4)
@@ -2769,17 +2772,17 @@ class LzEngine final : public LzEngineBase {
 #undef K1W
         if constexpr (B >= 4 && sizeof(XT) * 4 <= 16) {
             if (var == 4) {
-                hipLaunchKernelGGL((k_lz_a_rl<XT, B, 4, FMT>), g, dim3(LZ_WG), shm, s, a, rows, nv);
+                hipLaunchKernelGGL((k_lz_a_rl<XT, B, 4>), g, dim3(LZ_WG), k1_shm(4), s, a, rows, nv, tile_cap);
                 return;
             }
         }
         if constexpr (B >= 2) {
             if (var == 2) {
-                hipLaunchKernelGGL((k_lz_a_rl<XT, B, 2, FMT>), g, dim3(LZ_WG), shm, s, a, rows, nv);
+                hipLaunchKernelGGL((k_lz_a_rl<XT, B, 2>), g, dim3(LZ_WG), k1_shm(2), s, a, rows, nv, tile_cap);
                 return;
             }
         }
-        hipLaunchKernelGGL((k_lz_a_rl<XT, B, 1, FMT>), g, dim3(LZ_WG), shm, s, a, rows, nv);
+        hipLaunchKernelGGL((k_lz_a_rl<XT, B, 1>), g, dim3(LZ_WG), k1_shm(1), s, a, rows, nv, tile_cap);
     }
     void launch_k1(int LM) {
         const int nv = (1 + 2 * LM) * B;
@@ -3325,9 +3328,10 @@ class LzEngine final : public LzEngineBase {
     LzArgs<XT> a{};
     int k1v = 1, grid_rb = 1, grid_rl = 1, grid_k1 = 1, grid_k2 = 1;
     bool staged_ok = false, tuned = false;
-    int64_t rpw = 1, rpw_so = 1, nrblk = 0;
+    int64_t rpw_so = 1, nrblk = 0;
     const int32_t* rblk = nullptr;
     size_t shm = 0, shm_rb = 0;
+    int tile_cap = 0;
     std::vector<RunHost> rh;
     std::vector<int> act, nlock, jl, tot, kept, nextc;
     std::vector<int> jsync, totsync;  // step counts at the last analysis' device sync
@@ -3384,13 +3388,14 @@ size_t bh_engine_bytes(int64_t D, int prec, int B, const bh_lanczos_opts& o) {
     const bool fr = bh_lz_fullre(D, o);
     const size_t es = (prec == BH_PREC_FP64 || fr) ? 8 : 4;
     const size_t vs = static_cast<size_t>(D) * Bp;
-    const int64_t rpw = std::max<int64_t>(static_cast<int64_t>(LZ_WG / Bp) * LZ_K1_TILES, (D + LZ_K1_GRID_MAX - 1) / LZ_K1_GRID_MAX);
+    int64_t grid_rl = 1;
+    for (int V = 1; V <= std::min(Bp, 8); V *= 2) grid_rl = std::max(grid_rl, (D + lz_k1_rows(D, Bp, V) - 1) / lz_k1_rows(D, Bp, V));
     const int ymax = lz_ymax(D, o);
     const LzFrSplit frs = lz_fr_split(static_cast<int64_t>(vs), slots - 1, ymax);
     const size_t row_bytes = static_cast<size_t>(std::max(2 * LZ_NVMAX + 1 + 2 * LZ_LMAX, ymax)) * Bp * 8;
     // partial-sum rows: the row-lane and K2 grids, or the staged K1's (up to LZ_PART_BYTES)
     const size_t part_rows = std::max<size_t>(
-        static_cast<size_t>(std::max<int64_t>({LZ_GRID_MAX, LZ_K2_GRID, (D + rpw - 1) / rpw})),
+        static_cast<size_t>(std::max<int64_t>({LZ_GRID_MAX, LZ_K2_GRID, grid_rl})),
         std::min<size_t>(LZ_K1_GRID_MAX, static_cast<size_t>(LZ_PART_BYTES) / row_bytes));
     return (static_cast<size_t>(slots) + ymax + 1) * vs * es + vs * 8 + static_cast<size_t>(D) * 8 +
            part_rows * row_bytes +

@@ -4,23 +4,28 @@
 // (external/spectra/include/Spectra/MatOp/SparseGenMatProd.h:81-86 ->
 // include/Eigen/src/SparseCore/SparseDenseProduct.h:86-107), a serial column scatter in the
 // reference.  Here: CSR rows, G lanes per row and B vectors per CSR pass, FP64 accumulation.
-// The kernel is HBM-bound: per pass it reads the matrix once (4 B per entry in the packed format,
-// 12 B in FP64 CSR) plus the row pointers and the diagonal, and B * (x gather + y write).
+// Both precisions read the packed words and the exact FP64 values of the table; they differ in the vectors.
+// The kernel is HBM-bound: per pass it reads the matrix once (4 B per entry) plus the row pointers and the
+// diagonal, and B * (x gather + y write).
+#include <algorithm>
 #include <cmath>
 #include <mutex>
 
 #include "bh_kernels.hpp"
 #include "bh_spmv.hpp"
 
-template <typename XT, int B, int G, int FMT>
+template <int WG>
+__device__ __forceinline__ void spmv_table(const double* __restrict__ table, int cb, double* tab) {
+    for (int i = threadIdx.x; i < (1 << cb); i += WG) tab[i] = table[i];
+    __syncthreads();
+}
+
+template <typename XT, int B, int G>
 __global__ void __launch_bounds__(BH_WG) k_spmv(SpmvArgs<XT> a) {
     constexpr int GB = G * B;
     constexpr int SLOTS = BH_WG / GB;
-    extern __shared__ double tab[];  // (1 << cb) entries, packed format only
-    if constexpr (FMT == BH_FMT_PACKED) {
-        for (int i = threadIdx.x; i < (1 << a.cb); i += BH_WG) tab[i] = a.table[i];
-        __syncthreads();
-    }
+    extern __shared__ double tab[];  // (1 << cb) entries
+    spmv_table<BH_WG>(a.table, a.cb, tab);
     const int lane = threadIdx.x;
     const int slot = lane / GB;
     const int g = (lane % GB) / B;
@@ -30,116 +35,148 @@ __global__ void __launch_bounds__(BH_WG) k_spmv(SpmvArgs<XT> a) {
     if (tile >= ntile) return;  // whole workgroup leaves together (tile is uniform)
     const int64_t r = tile * SLOTS + slot;
     double acc = 0.0;
-    if (r < a.D) acc = bh_row_partial<XT, B, G, FMT>(a.row_ptr[r], a.row_ptr[r + 1], g, b, a.words, a.col64, a.val64, tab,
-                                                       a.cb, a.x);
+    if (r < a.D) acc = bh_row_partial<XT, B, G>(a.row_ptr[r], a.row_ptr[r + 1], g, b, a.words, tab, a.cb, a.x);
     acc = bh_group_sum<B, G>(acc);
     if (g == 0 && r < a.D) {
-        const double hx = (FMT == BH_FMT_PACKED) ? -acc : acc;
-        const double d = a.diag32 ? static_cast<double>(a.diag32[r]) : a.diag64[r];
         const double xr = to_d(a.x[r * B + b]);
-        a.y[r * B + b] = static_cast<XT>(a.J[b] * hx + a.U[b] * d * xr);
+        a.y[r * B + b] = static_cast<XT>(a.J[b] * -acc + a.U[b] * static_cast<double>(a.diag[r]) * xr);
     }
 }
 
-template <typename XT, int B, int FMT>
+template <typename XT, int B>
 __global__ void __launch_bounds__(BH_WG) k_spmv_rb(SpmvArgs<XT> a, const int32_t* __restrict__ rb, int64_t nblocks) {
     extern __shared__ double smem[];
-    double* tab = smem;                                  // (1 << cb) entries (packed format)
-    double* prod = smem + (FMT == BH_FMT_PACKED ? (1 << a.cb) : 0);
-    if constexpr (FMT == BH_FMT_PACKED) {
-        for (int i = threadIdx.x; i < (1 << a.cb); i += BH_WG) tab[i] = a.table[i];
-        __syncthreads();
-    }
+    double* tab = smem;  // (1 << cb) entries
+    double* prod = smem + (1 << a.cb);
+    spmv_table<BH_WG>(a.table, a.cb, tab);
     const int64_t t = a.xcd ? bh_xcd_tile(blockIdx.x, gridDim.x) : blockIdx.x;
     auto epi = [&](int64_t r, int bb, const double (&sum)[1]) {
-        const double hx = (FMT == BH_FMT_PACKED) ? -sum[0] : sum[0];
-        const double d = a.diag32 ? static_cast<double>(a.diag32[r]) : a.diag64[r];
-        a.y[r * B + bb] = static_cast<XT>(a.J[bb] * hx + a.U[bb] * d * to_d(a.x[r * B + bb]));
+        const double d = static_cast<double>(a.diag[r]);
+        a.y[r * B + bb] = static_cast<XT>(a.J[bb] * -sum[0] + a.U[bb] * d * to_d(a.x[r * B + bb]));
     };
-    bh_rowblock_run<XT, B, FMT, BH_WG>(t, t + 1, rb, a.row_ptr, a.words, a.col64, a.val64, tab, a.cb, a.x, prod, epi);
+    bh_rowblock_run<XT, B, BH_WG>(t, t + 1, rb, a.row_ptr, a.words, tab, a.cb, a.x, prod, epi);
 }
 
-template <typename XT, int B, int V, int FMT>
-__global__ void __launch_bounds__(BH_WG) k_spmv_rl(SpmvArgs<XT> a, int64_t rows_per_wg) {
-    extern __shared__ double tab[];
-    if constexpr (FMT == BH_FMT_PACKED) {
-        for (int i = threadIdx.x; i < (1 << a.cb); i += BH_WG) tab[i] = a.table[i];
-        __syncthreads();
-    }
-    const int64_t t = a.xcd ? bh_xcd_tile(blockIdx.x, gridDim.x) : blockIdx.x;
-    const int64_t r0 = min(t * rows_per_wg, a.D), r1 = min(r0 + rows_per_wg, a.D);
-    auto epi = [&](int64_t r, int b0, const double (&acc)[V]) {
-        const double d = a.diag32 ? static_cast<double>(a.diag32[r]) : a.diag64[r];
+// epilogue of the row-lane and row-tile engines: y for the V vectors a thread holds of a row
+template <typename XT, int B, int V>
+struct SpmvEpi {
+    const SpmvArgs<XT>& a;
+    __device__ __forceinline__ void operator()(int64_t r, int b0, const double (&acc)[V]) const {
+        const double d = static_cast<double>(a.diag[r]);
         const BhVec<XT, V> xv = bh_vload<V>(a.x + r * B + b0);
         BhVec<XT, V> yv;
 #pragma unroll
-        for (int v = 0; v < V; ++v) {
-            const double hx = (FMT == BH_FMT_PACKED) ? -acc[v] : acc[v];
-            yv.v[v] = static_cast<XT>(a.J[b0 + v] * hx + a.U[b0 + v] * d * to_d(xv.v[v]));
-        }
+        for (int v = 0; v < V; ++v)
+            yv.v[v] = static_cast<XT>(a.J[b0 + v] * -acc[v] + a.U[b0 + v] * d * to_d(xv.v[v]));
         *reinterpret_cast<BhVec<XT, V>*>(a.y + r * B + b0) = yv;
-    };
-    bh_rowlane_run<XT, B, V, FMT, BH_WG, 4>(r0, r1, a.row_ptr, a.words, a.col64, a.val64, tab, a.cb, a.x, epi);
+    }
+};
+
+template <typename XT, int B, int V>
+__global__ void __launch_bounds__(BH_WG) k_spmv_rl(SpmvArgs<XT> a, int64_t rows_per_wg) {
+    extern __shared__ double tab[];
+    spmv_table<BH_WG>(a.table, a.cb, tab);
+    const int64_t t = a.xcd ? bh_xcd_tile(blockIdx.x, gridDim.x) : blockIdx.x;
+    const int64_t r0 = min(t * rows_per_wg, a.D), r1 = min(r0 + rows_per_wg, a.D);
+    SpmvEpi<XT, B, V> epi{a};
+    bh_rowlane_run<XT, B, V, BH_WG, 4>(r0, r1, a.row_ptr, a.words, tab, a.cb, a.x, epi);
 }
 
-// row-lane engine with V vectors per thread (V * sizeof(XT) <= 16 bytes, V <= B)
-template <typename XT, int FMT>
-static void launch_spmv_rl_t(const SpmvArgs<XT>& a, int B, int V, hipStream_t s) {
-    const size_t shm = FMT == BH_FMT_PACKED ? (static_cast<size_t>(1) << a.cb) * sizeof(double) : 0;
-    const int64_t rows_per_wg = static_cast<int64_t>(BH_WG) * V / B * 4;
+// one thread per row (V = B): the words of a wave's 64 rows go through LDS
+template <typename XT, int V>
+__global__ void __launch_bounds__(BH_WG) k_spmv_rt(SpmvArgs<XT> a, int64_t rows_per_wg, int cap) {
+    extern __shared__ __align__(16) double smem[];
+    double* tab = smem;
+    spmv_table<BH_WG>(a.table, a.cb, tab);
+    const int64_t t = a.xcd ? bh_xcd_tile(blockIdx.x, gridDim.x) : blockIdx.x;
+    const int64_t r0 = min(t * rows_per_wg, a.D), r1 = min(r0 + rows_per_wg, a.D);
+    SpmvEpi<XT, V, V> epi{a};
+    bh_rowtile_run<XT, V, BH_WG, (V == 1 ? 8 : 4)>(r0, r1, a.row_ptr, a.words, tab, a.cb, a.x,
+                                                   reinterpret_cast<uint32_t*>(smem + (1 << a.cb)), cap, epi);
+}
+
+int bh_tile_cap(const bh_ham* h) {
+    const int need = 64 * std::max(h->max_row, 1) + 8;
+    return std::min((need + 63) / 64 * 64, BH_TILE_WORDS);
+}
+
+// row-lane engine with V vectors per thread (V * sizeof(XT) <= 16 bytes, V <= B); one thread per row: row tiles
+template <typename XT>
+static void launch_spmv_rl(const bh_ham* h, const SpmvArgs<XT>& a, int B, int V, hipStream_t s) {
+    const size_t shm = (static_cast<size_t>(1) << a.cb) * sizeof(double);
+    // up to four passes of BH_WG V / B rows per workgroup, fewer while that leaves under 1024 workgroups (four per CU)
+    const int64_t pass = static_cast<int64_t>(BH_WG) * V / B;
+    const int64_t rows_per_wg = pass * std::max<int64_t>(1, std::min<int64_t>(4, a.D / (pass * 1024)));
     const unsigned grid = static_cast<unsigned>((a.D + rows_per_wg - 1) / rows_per_wg);
-#define L(BB, VV)                                                                                              \
+    if (B == V) {
+        const int cap = bh_tile_cap(h);
+        const size_t sht = shm + static_cast<size_t>(BH_WG / 64) * cap * sizeof(uint32_t);
+        if (V == 1) hipLaunchKernelGGL((k_spmv_rt<XT, 1>), dim3(grid), dim3(BH_WG), sht, s, a, rows_per_wg, cap);
+        else if (V == 2) hipLaunchKernelGGL((k_spmv_rt<XT, 2>), dim3(grid), dim3(BH_WG), sht, s, a, rows_per_wg, cap);
+        if constexpr (sizeof(XT) == 4)
+            if (V == 4) hipLaunchKernelGGL((k_spmv_rt<XT, 4>), dim3(grid), dim3(BH_WG), sht, s, a, rows_per_wg, cap);
+        return;
+    }
+#define L(BB, VV)                                                                                             \
     if (B == BB && V == VV) {                                                                                 \
-        hipLaunchKernelGGL((k_spmv_rl<XT, BB, VV, FMT>), dim3(grid), dim3(BH_WG), shm, s, a, rows_per_wg);    \
+        hipLaunchKernelGGL((k_spmv_rl<XT, BB, VV>), dim3(grid), dim3(BH_WG), shm, s, a, rows_per_wg);         \
         return;                                                                                               \
     }
-    L(1, 1) L(2, 1) L(4, 1) L(8, 1) L(16, 1) L(32, 1) L(64, 1)
-    L(2, 2) L(4, 2) L(8, 2) L(16, 2) L(32, 2) L(64, 2)
+    L(2, 1) L(4, 1) L(8, 1) L(16, 1) L(32, 1) L(64, 1)
+    L(4, 2) L(8, 2) L(16, 2) L(32, 2) L(64, 2)
     if constexpr (sizeof(XT) == 4) {
-        L(4, 4) L(8, 4) L(16, 4) L(32, 4) L(64, 4)
+        L(8, 4) L(16, 4) L(32, 4) L(64, 4)
     }
 #undef L
 }
 
-template <typename XT, int FMT>
-static void launch_spmv_rb_t(const SpmvArgs<XT>& a, int B, const int32_t* rb, int64_t nb, hipStream_t s) {
-    const size_t shm = ((FMT == BH_FMT_PACKED ? (static_cast<size_t>(1) << a.cb) : 0) + BH_STAGE_PRODUCTS) * sizeof(double);
+template <typename XT>
+static void launch_spmv_rb(const SpmvArgs<XT>& a, int B, const int32_t* rb, int64_t nb, hipStream_t s) {
+    const size_t shm = ((static_cast<size_t>(1) << a.cb) + BH_STAGE_PRODUCTS) * sizeof(double);
     const unsigned grid = static_cast<unsigned>(nb);
-#define L(BB)                                                                                            \
-    if (B == BB) {                                                                                      \
-        hipLaunchKernelGGL((k_spmv_rb<XT, BB, FMT>), dim3(grid), dim3(BH_WG), shm, s, a, rb, nb);       \
-        return;                                                                                         \
+#define L(BB)                                                                                       \
+    if (B == BB) {                                                                                  \
+        hipLaunchKernelGGL((k_spmv_rb<XT, BB>), dim3(grid), dim3(BH_WG), shm, s, a, rb, nb);        \
+        return;                                                                                     \
     }
     L(1) L(2) L(4) L(8) L(16) L(32) L(64)
 #undef L
 }
 
-void bh_launch_spmv_rb(const SpmvArgs<float>& a, int B, const int32_t* rb, int64_t nb, hipStream_t s) {
-    launch_spmv_rb_t<float, BH_FMT_PACKED>(a, B, rb, nb, s);
-}
-void bh_launch_spmv_rb(const SpmvArgs<double>& a, int B, int fmt, const int32_t* rb, int64_t nb, hipStream_t s) {
-    if (fmt == BH_FMT_PACKED) launch_spmv_rb_t<double, BH_FMT_PACKED>(a, B, rb, nb, s);
-    else launch_spmv_rb_t<double, BH_FMT_CSR64>(a, B, rb, nb, s);
+template <typename XT>
+static void launch_spmv_g(const SpmvArgs<XT>& a, int B, int G, hipStream_t s) {
+    const int GB = G * B;
+    const int64_t slots = BH_WG / GB;
+    const unsigned grid = static_cast<unsigned>((a.D + slots - 1) / slots);
+    const size_t shm = (static_cast<size_t>(1) << a.cb) * sizeof(double);
+#define L(BB, GG)                                                                          \
+    if (B == BB && G == GG) {                                                              \
+        hipLaunchKernelGGL((k_spmv<XT, BB, GG>), dim3(grid), dim3(BH_WG), shm, s, a);      \
+        return;                                                                            \
+    }
+    L(1, 1) L(1, 2) L(1, 4) L(1, 8) L(1, 16) L(1, 32) L(1, 64)
+    L(2, 1) L(2, 2) L(2, 4) L(2, 8) L(2, 16) L(2, 32)
+    L(4, 1) L(4, 2) L(4, 4) L(4, 8) L(4, 16)
+    L(8, 1) L(8, 2) L(8, 4) L(8, 8)
+    L(16, 1) L(16, 2) L(16, 4)
+    L(32, 1) L(32, 2)
+    L(64, 1)
+#undef L
 }
 
-// SpMV variants: 0 = LDS-staged row blocks; V = 1, 2, 4 = row-lane engine with V vectors per thread
-// (64 V / B rows per wavefront); 100 + G = G lanes per row (64 / (G B) rows per wavefront)
-static int spmv_launch(bh_ham* h, int var, const SpmvArgs<double>* a64, const SpmvArgs<float>* a32, int fmt, int B,
-                       hipStream_t s) {
+// SpMV variants: 0 = LDS-staged row blocks; V = 1, 2, 4 = V vectors per thread, B / V threads per row (64 V / B
+// rows per wavefront); 100 + G = G lanes per row (64 / (G B) rows per wavefront)
+template <typename XT>
+static int spmv_launch(bh_ham* h, int var, const SpmvArgs<XT>& a, int B, hipStream_t s) {
     if (var == 0) {
         const int32_t* rb = nullptr;
         int64_t nb = 0;
         BH_TRY(bh_ham_rowblocks(h, B, &rb, &nb));
-        if (a64) bh_launch_spmv_rb(*a64, B, fmt, rb, nb, s);
-        else bh_launch_spmv_rb(*a32, B, rb, nb, s);
+        launch_spmv_rb(a, B, rb, nb, s);
     } else if (var >= 100) {
-        if (a64) bh_launch_spmv(*a64, B, var - 100, fmt, s);
-        else bh_launch_spmv(*a32, B, var - 100, s);
-    } else if (a64) {
-        if (fmt == BH_FMT_PACKED) launch_spmv_rl_t<double, BH_FMT_PACKED>(*a64, B, var, s);
-        else launch_spmv_rl_t<double, BH_FMT_CSR64>(*a64, B, var, s);
+        launch_spmv_g(a, B, var - 100, s);
     } else {
-        launch_spmv_rl_t<float, BH_FMT_PACKED>(*a32, B, var, s);
+        launch_spmv_rl(h, a, B, var, s);
     }
     return BH_OK;
 }
@@ -148,25 +185,24 @@ static int spmv_launch(bh_ham* h, int var, const SpmvArgs<double>* a64, const Sp
 // (precision, B) runs the autotuner unless BHX_TUNE=0 or BHX_ENGINE is set: every variant that fits is
 // timed with HIP events over a warm-up and three applications to the caller's own x and y (y = H x is
 // idempotent), and the fastest is kept in the handle.  Under stream capture the default variant is used.
-int bh_apply(bh_ctx* ctx, bh_ham* h, const SpmvArgs<double>* a64, const SpmvArgs<float>* a32, int fmt, int B,
-             hipStream_t s) {
-    const int prec = a32 ? BH_PREC_MIXED : (fmt == BH_FMT_CSR64 ? BH_PREC_FP64 : 2);
+template <typename XT>
+static int apply_t(bh_ctx* ctx, bh_ham* h, const SpmvArgs<XT>& a, int prec, int B, hipStream_t s) {
     const int key = bh_tune_key(1, prec, B);
     std::lock_guard<std::recursive_mutex> lk(ctx->mu);
     auto it = h->tuned.find(key);
-    if (it != h->tuned.end()) return spmv_launch(h, it->second.variant, a64, a32, fmt, B, s);
+    if (it != h->tuned.end()) return spmv_launch(h, it->second.variant, a, B, s);
     const int eng = bh_engine_choice(B, h);
     BhTuned t;
     t.variant = eng == 2 ? 1 : (eng == 1 ? 0 : 100 + bh_pick_lanes(h, B));
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     BH_HIP(ctx, hipStreamIsCapturing(s, &cs));
-    if (cs != hipStreamCaptureStatusNone) return spmv_launch(h, t.variant, a64, a32, fmt, B, s);
+    if (cs != hipStreamCaptureStatusNone) return spmv_launch(h, t.variant, a, B, s);
     if (bh_tune_enabled() && bh_engine_env() < 0) {
         std::vector<int> cand;
         if (static_cast<int64_t>(h->max_row) * B <= BH_STAGE_PRODUCTS_HOST) cand.push_back(0);
         cand.push_back(1);
         if (B >= 2) cand.push_back(2);
-        if (B >= 4 && a32) cand.push_back(4);
+        if (B >= 4 && sizeof(XT) == 4) cand.push_back(4);
         const int G = bh_pick_lanes(h, B);
         if (G > 1) cand.push_back(100 + G);
         hipEvent_t e0 = nullptr, e1 = nullptr;
@@ -174,9 +210,9 @@ int bh_apply(bh_ctx* ctx, bh_ham* h, const SpmvArgs<double>* a64, const SpmvArgs
         BH_HIP(ctx, hipEventCreate(&e1));
         double best = 0.0;
         for (int var : cand) {
-            BH_TRY(spmv_launch(h, var, a64, a32, fmt, B, s));
+            BH_TRY(spmv_launch(h, var, a, B, s));
             BH_HIP(ctx, hipEventRecord(e0, s));
-            for (int r = 0; r < 3; ++r) BH_TRY(spmv_launch(h, var, a64, a32, fmt, B, s));
+            for (int r = 0; r < 3; ++r) BH_TRY(spmv_launch(h, var, a, B, s));
             BH_HIP(ctx, hipEventRecord(e1, s));
             BH_HIP(ctx, hipEventSynchronize(e1));
             float ms = 0.f;
@@ -192,34 +228,14 @@ int bh_apply(bh_ctx* ctx, bh_ham* h, const SpmvArgs<double>* a64, const SpmvArgs
         (void)hipEventDestroy(e1);
     }
     h->tuned[key] = t;
-    return spmv_launch(h, t.variant, a64, a32, fmt, B, s);
+    return spmv_launch(h, t.variant, a, B, s);
 }
 
-template <typename XT, int FMT>
-static void launch_spmv_t(const SpmvArgs<XT>& a, int B, int G, hipStream_t s) {
-    const int GB = G * B;
-    const int64_t slots = BH_WG / GB;
-    const unsigned grid = static_cast<unsigned>((a.D + slots - 1) / slots);
-    const size_t shm = FMT == BH_FMT_PACKED ? (static_cast<size_t>(1) << a.cb) * sizeof(double) : 0;
-#define L(BB, GG)                                                                               \
-    if (B == BB && G == GG) {                                                                  \
-        hipLaunchKernelGGL((k_spmv<XT, BB, GG, FMT>), dim3(grid), dim3(BH_WG), shm, s, a);     \
-        return;                                                                                \
-    }
-    L(1, 1) L(1, 2) L(1, 4) L(1, 8) L(1, 16) L(1, 32) L(1, 64)
-    L(2, 1) L(2, 2) L(2, 4) L(2, 8) L(2, 16) L(2, 32)
-    L(4, 1) L(4, 2) L(4, 4) L(4, 8) L(4, 16)
-    L(8, 1) L(8, 2) L(8, 4) L(8, 8)
-    L(16, 1) L(16, 2) L(16, 4)
-    L(32, 1) L(32, 2)
-    L(64, 1)
-#undef L
+int bh_apply(bh_ctx* ctx, bh_ham* h, const SpmvArgs<double>& a, int key, int B, hipStream_t s) {
+    return apply_t(ctx, h, a, key, B, s);
 }
-
-void bh_launch_spmv(const SpmvArgs<float>& a, int B, int G, hipStream_t s) { launch_spmv_t<float, BH_FMT_PACKED>(a, B, G, s); }
-void bh_launch_spmv(const SpmvArgs<double>& a, int B, int G, int fmt, hipStream_t s) {
-    if (fmt == BH_FMT_PACKED) launch_spmv_t<double, BH_FMT_PACKED>(a, B, G, s);
-    else launch_spmv_t<double, BH_FMT_CSR64>(a, B, G, s);
+int bh_apply(bh_ctx* ctx, bh_ham* h, const SpmvArgs<float>& a, int key, int B, hipStream_t s) {
+    return apply_t(ctx, h, a, key, B, s);
 }
 
 int bh_pick_lanes(const bh_ham* h, int B) {
@@ -233,8 +249,7 @@ int bh_pick_lanes(const bh_ham* h, int B) {
 
 double bh_spmv_bytes(const bh_ham* h, int prec, int B) {
     const double D = static_cast<double>(h->D), nnz = static_cast<double>(h->nnz);
-    if (prec == BH_PREC_FP64) return nnz * 12.0 + 4.0 * (D + 1) + 8.0 * D + B * 2.0 * 8.0 * D;
-    return nnz * 4.0 + 4.0 * (D + 1) + 4.0 * D + B * 2.0 * 4.0 * D;
+    return nnz * 4.0 + 4.0 * (D + 1) + 4.0 * D + B * 2.0 * (prec == BH_PREC_FP64 ? 8.0 : 4.0) * D;
 }
 
 int bh_is_pow2_le64(int B) { return B >= 1 && B <= 64 && (B & (B - 1)) == 0; }
@@ -277,8 +292,8 @@ int bh_spmv_noalloc(bh_ctx* ctx, bh_ham* h, int prec, int B, const double* J, co
     if (prec != BH_PREC_FP64 && prec != BH_PREC_MIXED) return bh_set_error(ctx, BH_EINVAL, "spmv_noalloc: prec");
     std::lock_guard<std::recursive_mutex> lk(ctx->mu);
     BH_HIP(ctx, hipSetDevice(ctx->device));
-    if (prec == BH_PREC_FP64 && !h->col64)
-        return bh_set_error(ctx, BH_EINVAL, "spmv_noalloc: FP64 CSR not materialised (bh_ham_prepare first)");
+    if (prec == BH_PREC_FP64 && !h->prepared64)
+        return bh_set_error(ctx, BH_EINVAL, "spmv_noalloc: handle not prepared for FP64 (bh_ham_prepare first)");
     hipStream_t s = stream ? static_cast<hipStream_t>(stream) : ctx->stream;
     double* sc = nullptr;
     BH_TRY(scratch_ptr(ctx, &sc));
@@ -297,13 +312,13 @@ int bh_spmv_noalloc(bh_ctx* ctx, bh_ham* h, int prec, int B, const double* J, co
     }
     if (var == 0 && h->rowblocks.find(B) == h->rowblocks.end()) var = 1;
     if (prec == BH_PREC_FP64) {
-        SpmvArgs<double> a{h->D, h->row_ptr, h->words, h->col64, h->val64, nullptr, h->diag64, h->table, h->code_bits,
+        SpmvArgs<double> a{h->D, h->row_ptr, h->words, h->diag, h->table, h->code_bits,
                            sc, sc + SPMV_SCRATCH_LANES, static_cast<const double*>(x), static_cast<double*>(y), 1};
-        BH_TRY(spmv_launch(h, var, &a, nullptr, BH_FMT_CSR64, B, s));
+        BH_TRY(spmv_launch(h, var, a, B, s));
     } else {
-        SpmvArgs<float> a{h->D, h->row_ptr, h->words, nullptr, nullptr, h->diag, nullptr, h->table, h->code_bits,
+        SpmvArgs<float> a{h->D, h->row_ptr, h->words, h->diag, h->table, h->code_bits,
                           sc, sc + SPMV_SCRATCH_LANES, static_cast<const float*>(x), static_cast<float*>(y), 1};
-        BH_TRY(spmv_launch(h, var, nullptr, &a, BH_FMT_PACKED, B, s));
+        BH_TRY(spmv_launch(h, var, a, B, s));
     }
     BH_HIP(ctx, hipGetLastError());
     // outside a capture the call returns with its work done (the host's J and U may be reused at once)
@@ -329,13 +344,13 @@ int bh_spmv(bh_ctx* ctx, bh_ham* h, int prec, int B, const double* J, const doub
     {
         KTimer kt(ctx, "spmv", s);
         if (prec == BH_PREC_FP64) {
-            SpmvArgs<double> a{h->D, h->row_ptr, h->words, h->col64, h->val64, nullptr, h->diag64, h->table, h->code_bits,
+            SpmvArgs<double> a{h->D, h->row_ptr, h->words, h->diag, h->table, h->code_bits,
                                dJ.p, dU.p, static_cast<const double*>(x), static_cast<double*>(y), 1};
-            BH_TRY(bh_apply(ctx, h, &a, nullptr, BH_FMT_CSR64, B, s));
+            BH_TRY(bh_apply(ctx, h, a, prec, B, s));
         } else {
-            SpmvArgs<float> a{h->D, h->row_ptr, h->words, nullptr, nullptr, h->diag, nullptr, h->table, h->code_bits,
+            SpmvArgs<float> a{h->D, h->row_ptr, h->words, h->diag, h->table, h->code_bits,
                               dJ.p, dU.p, static_cast<const float*>(x), static_cast<float*>(y), 1};
-            BH_TRY(bh_apply(ctx, h, nullptr, &a, BH_FMT_PACKED, B, s));
+            BH_TRY(bh_apply(ctx, h, a, prec, B, s));
         }
     }
     BH_HIP(ctx, hipGetLastError());
@@ -395,13 +410,13 @@ int bh_spmv_bench(bh_ctx* ctx, bh_ham* h, int prec, int B, int reps, double* avg
     BH_HIP(ctx, hipMemsetAsync(dx.p, 0, n * es, s));
     auto launch = [&]() -> int {
         if (prec == BH_PREC_FP64) {
-            SpmvArgs<double> a{h->D, h->row_ptr, h->words, h->col64, h->val64, nullptr, h->diag64, h->table, h->code_bits,
+            SpmvArgs<double> a{h->D, h->row_ptr, h->words, h->diag, h->table, h->code_bits,
                                dJ.p, dU.p, reinterpret_cast<const double*>(dx.p), reinterpret_cast<double*>(dy.p), 1};
-            return bh_apply(ctx, h, &a, nullptr, BH_FMT_CSR64, B, s);
+            return bh_apply(ctx, h, a, prec, B, s);
         }
-        SpmvArgs<float> a{h->D, h->row_ptr, h->words, nullptr, nullptr, h->diag, nullptr, h->table, h->code_bits,
+        SpmvArgs<float> a{h->D, h->row_ptr, h->words, h->diag, h->table, h->code_bits,
                           dJ.p, dU.p, reinterpret_cast<const float*>(dx.p), reinterpret_cast<float*>(dy.p), 1};
-        return bh_apply(ctx, h, nullptr, &a, BH_FMT_PACKED, B, s);
+        return bh_apply(ctx, h, a, prec, B, s);
     };
     BH_TRY(launch());  // warm-up (also builds the row blocks)
     hipEvent_t e0, e1;

@@ -9,11 +9,8 @@ template <typename XT>
 struct SpmvArgs {
     int64_t D;
     const int32_t* row_ptr;
-    const uint32_t* words;  // packed format
-    const int32_t* col64;   // FP64 CSR
-    const double* val64;
-    const float* diag32;    // one of diag32 / diag64
-    const double* diag64;
+    const uint32_t* words;  // column << cb | code
+    const float* diag;      // V (small integers and halves: exact)
     const double* table;    // sqrt(code)
     int cb;
     const double* J;        // [B]
@@ -23,13 +20,15 @@ struct SpmvArgs {
     int xcd;                // XCD-aware tile order
 };
 
-void bh_launch_spmv(const SpmvArgs<float>& a, int B, int G, hipStream_t s);
-void bh_launch_spmv(const SpmvArgs<double>& a, int B, int G, int fmt, hipStream_t s);
+// tuning keys of the operator pass: the caller's FP64 and mixed products, and the FP64 product of the solver's finish
+constexpr int BH_KEY_FINISH = 2;
+
 int bh_pick_lanes(const bh_ham* h, int B);
 double bh_spmv_bytes(const bh_ham* h, int prec, int B);
 int bh_is_pow2_le64(int B);
 int bh_ham_prepare_locked(bh_ham* h, int prec);
-void bh_launch_spmv_rb(const SpmvArgs<float>& a, int B, const int32_t* rb, int64_t nb, hipStream_t s);
-void bh_launch_spmv_rb(const SpmvArgs<double>& a, int B, int fmt, const int32_t* rb, int64_t nb, hipStream_t s);
-int bh_apply(bh_ctx* ctx, bh_ham* h, const SpmvArgs<double>* a64, const SpmvArgs<float>* a32, int fmt, int B,
-             hipStream_t s);
+// one product with the variant tuned for (h, key, B); key: BH_PREC_FP64, BH_PREC_MIXED or BH_KEY_FINISH
+int bh_apply(bh_ctx* ctx, bh_ham* h, const SpmvArgs<double>& a, int key, int B, hipStream_t s);
+int bh_apply(bh_ctx* ctx, bh_ham* h, const SpmvArgs<float>& a, int key, int B, hipStream_t s);
+// words of a wave's LDS part on the row-tile engine: the longest 64 rows could need, within BH_TILE_WORDS
+int bh_tile_cap(const bh_ham* h);

@@ -59,9 +59,8 @@ extern "C" {
 #define BH_ORDER_BAND 4
 
 /* ---- precisions --------------------------------------------------------------------------------- */
-/* BH_PREC_FP64: FP64 vectors and arithmetic -- the plain comparator.  The SpMV entry points read an FP64
- *   CSR (double value + int32 column); the Lanczos engine reads the packed words below, whose FP64 table
- *   gives the same exact values in 4 bytes per entry.
+/* BH_PREC_FP64: FP64 vectors and arithmetic -- the plain comparator.  It reads the packed words below, whose FP64
+ *   table gives the exact values in 4 bytes per entry.
  * BH_PREC_MIXED: one 32-bit word per entry (column << code_bits | code), value = -sqrt(code) read
  *   from an exact FP64 table, FP32-stored vectors, FP64 accumulation and reductions, FP64 finish. */
 #define BH_PREC_FP64 0
@@ -158,8 +157,8 @@ int64_t bh_ham_device_bytes(const bh_ham* h);
 int bh_ham_copy_csr(const bh_ham* h, int64_t* row_ptr, int32_t* col, double* val, double* diag);
 /* the packed words (column << code_bits | code) and code_bits of the mixed format */
 int bh_ham_copy_packed(const bh_ham* h, uint32_t* words, int* code_bits);
-/* Materialise the FP64 CSR of the FP64 SpMV entry points (needed once before their BH_PREC_FP64 use, and before
- * bh_spmv_noalloc in FP64; done lazily by bh_spmv otherwise; the Lanczos engines do not use it). */
+/* Prepares the handle for a precision: needed once before bh_spmv_noalloc in FP64 (bh_spmv and bh_spmv_host do it
+ * themselves).  Both precisions read the packed words, so nothing is allocated. */
 int bh_ham_prepare(bh_ham* h, int prec);
 /* No counterpart in the reference (its product has one fixed kernel): the operator-kernel variant the
  * autotuner chose for this sector at (kind, prec, B), once the sector has been used that way (kind 0: the
