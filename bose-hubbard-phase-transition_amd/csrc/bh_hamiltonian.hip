@@ -1,4 +1,4 @@
-// bh_hamiltonian.hip -- two-pass (count / exclusive scan / fill) CSR build of the hopping term T and
+// bh_hamiltonian.hip -- count / tile scan / fill CSR build of the hopping term T and
 // the diagonal interaction V over a neighbour list, in the basis order of a bh_basis.
 //
 // Reference: BH::fill_hopping (src/hamiltonian.cpp:170-191) and BH::fill_interaction (:194-211),
@@ -58,65 +58,220 @@ __device__ __forceinline__ int64_t pstate_rank(const PState<NW, BITS>& t, int m,
     return r;
 }
 
+// entries a row gains per occupied site: the distinct directed bonds that leave it
+struct SiteDeg {
+    uint8_t d[BH_MAX_SITES];
+};
+
+constexpr int HC_BLOCK = 256;
+constexpr int HC_TILE = 512;  // rows of a count tile (two per thread)
+
+// entries of every row (cnt) and of every tile of HC_TILE rows (tile)
 template <int NW, int BITS>
-__global__ void __launch_bounds__(HB_BLOCK) k_ham_count(int64_t D, int m, int n, const uint32_t* __restrict__ g,
-                                                         const int32_t* __restrict__ lex_of_pos, EdgeArgs ed,
-                                                         int32_t* __restrict__ rownnz) {
-    const int64_t q = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (q >= D) return;
-    PState<NW, BITS> s;
-    bh_unrank(lex_of_pos[q], m, n, g, s);
-    int c = 0;
-    for (int e = 0; e < ed.E; ++e) c += s.get(ed.ej[e]) >= 1;
-    rownnz[q] = c;
+__global__ void __launch_bounds__(HC_BLOCK) k_ham_count(int64_t D, int m, int n, const uint32_t* __restrict__ gg, int gsize,
+                                                        const int32_t* __restrict__ lex_of_pos, SiteDeg deg,
+                                                        uint8_t* __restrict__ cnt, int64_t* __restrict__ tile) {
+    extern __shared__ uint32_t g[];
+    __shared__ int red[HC_BLOCK / 64];
+    bh_stage_table(gg, gsize, g);
+    int sum = 0;
+#pragma unroll
+    for (int u = 0; u < HC_TILE / HC_BLOCK; ++u) {
+        const int64_t q = static_cast<int64_t>(blockIdx.x) * HC_TILE + u * HC_BLOCK + threadIdx.x;
+        if (q >= D) continue;
+        PState<NW, BITS> s;
+        bh_unrank(lex_of_pos[q], m, n, g, s);
+        int c = 0;
+#pragma unroll
+        for (int j = 0; j < PState<NW, BITS>::MAXM; ++j)
+            if (j < m) c += s.get(j) >= 1 ? deg.d[j] : 0;
+        cnt[q] = static_cast<uint8_t>(c);
+        sum += c;
+    }
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) sum += __shfl_xor(sum, o, 64);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = sum;
+    __syncthreads();
+    if (threadIdx.x == 0) tile[blockIdx.x] = red[0] + red[1] + red[2] + red[3];
 }
 
-template <int NW, int BITS>
-__global__ void __launch_bounds__(HB_BLOCK) k_ham_fill(int64_t D, int m, int n, const uint32_t* __restrict__ g_glob,
-                                                        int gsize, const int32_t* __restrict__ lex_of_pos,
-                                                        const int32_t* __restrict__ pos_of_lex, EdgeArgs ed, int cb,
-                                                        unsigned flags, const int32_t* __restrict__ row_ptr,
-                                                        uint32_t* __restrict__ words, float* __restrict__ diag) {
-    extern __shared__ uint32_t lds[];
-    uint32_t* g = lds;                                   // gsize words
-    const int stride = ed.E + 1;                         // odd stride: no LDS bank aliasing between lanes
-    uint32_t* ent = lds + gsize + threadIdx.x * stride;  // this thread's row buffer
-    for (int a = threadIdx.x; a < gsize; a += blockDim.x) g[a] = g_glob[a];
-    __syncthreads();
-    const int64_t q = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (q >= D) return;
-    PState<NW, BITS> s;
-    bh_unrank(lex_of_pos[q], m, n, g, s);
-    int cnt = 0;
-    for (int e = 0; e < ed.E; ++e) {
-        const int i = ed.ei[e], j = ed.ej[e];
-        const int nj = s.get(j);
-        if (nj < 1) continue;
-        const int ni = s.get(i);
-        PState<NW, BITS> t = s;
-        pstate_add(t, i, 1);
-        pstate_add(t, j, -1);
-        const int64_t tl = pstate_rank(t, m, n, g);
-        const uint32_t col = static_cast<uint32_t>(pos_of_lex[tl]);
-        const uint32_t code = ed.cm[e] * static_cast<uint32_t>((ni + 1) * nj);
-        // insertion into the sorted row buffer (distinct targets: distinct (i,j) pairs)
-        const uint32_t wv = (col << cb) | code;
-        int a = cnt - 1;
-        while (a >= 0 && ent[a] > wv) {
-            ent[a + 1] = ent[a];
-            --a;
-        }
-        ent[a + 1] = wv;
-        ++cnt;
+// single workgroup: exclusive scan of the nb tile sums in place
+__global__ void __launch_bounds__(1024) k_scan_tiles(int64_t* __restrict__ tile, int64_t nb) {
+    __shared__ int64_t lds[1024 / 64 + 1];
+    const int64_t per = (nb + 1023) / 1024;
+    const int64_t b0 = static_cast<int64_t>(threadIdx.x) * per;
+    int64_t s = 0;
+    for (int64_t i = b0; i < b0 + per && i < nb; ++i) s += tile[i];
+    int64_t run = bh_block_exclusive_scan<1024>(s, lds, nullptr);
+    for (int64_t i = b0; i < b0 + per && i < nb; ++i) {
+        const int64_t t = tile[i];
+        tile[i] = run;
+        run += t;
     }
-    const int32_t base = row_ptr[q];
-    for (int a = 0; a < cnt; ++a) words[base + a] = ent[a];
+}
+
+// w[0 .. P-1] ascending: Batcher's odd-even merge sort, every index known at compile time (registers)
+template <int P>
+__device__ __forceinline__ void sort_registers(uint32_t (&w)[P]) {
+#pragma unroll
+    for (int p = 1; p < P; p <<= 1)
+#pragma unroll
+        for (int k = p; k >= 1; k >>= 1)
+#pragma unroll
+            for (int j = k % p; j + k < P; j += 2 * k)
+#pragma unroll
+                for (int i = 0; i < k; ++i)
+                    if (i + j + k < P && (i + j) / (2 * p) == (i + j + k) / (2 * p)) {
+                        const uint32_t a = w[i + j], b = w[i + j + k];
+                        w[i + j] = min(a, b);
+                        w[i + j + k] = max(a, b);
+                    }
+}
+
+// Fill, one wave per 64 rows: row pointers, sorted words, diagonal, and the wave's part of the row statistics.
+// A thread unranks its row's state once and keeps, for every site l, the sums over l' < l of the steps
+// g[l'][R] - g[l'][R - 1] and g[l'][R + 1] - g[l'][R] (R: bosons right of l'); moving a boson from j to i changes R by one
+// on the sites between, so a hop's rank is the row's plus one difference of two such sums, whatever the
+// distance.  Every directed bond has a register (P >= E of them; all ones where its source is empty, which no entry
+// is: the word of D = 2^k states only), so that the gathers of the positions are in flight together and the row
+// is sorted by a network of min / max instead of an insertion whose 64 lanes wait for the longest (P = 32: 191 pairs).
+// The 64 rows are one contiguous run of words: they are laid out in LDS and written coalesced.  D = 1,352,078 with E = 24 bonds
+// in the reference's order: 280 -> 191 us, now bound by the gathers of the positions (5.4 MB, more than one L2).
+// stats: longest row, largest row sum of |T|, min and max of V.
+template <int NW, int BITS, int P>
+__global__ void __launch_bounds__(HB_BLOCK) k_ham_fill(int64_t D, int m, int n, const uint32_t* __restrict__ g_glob, int gsize,
+                                                       const int32_t* __restrict__ lex_of_pos,
+                                                       const int32_t* __restrict__ pos_of_lex, EdgeArgs ed, int cb,
+                                                       const double* __restrict__ table, unsigned flags,
+                                                       const uint8_t* __restrict__ cntg, const int64_t* __restrict__ tile,
+                                                       int64_t nnz, int32_t* __restrict__ row_ptr, uint32_t* __restrict__ words,
+                                                       float* __restrict__ diag, int4* __restrict__ stats) {
+    extern __shared__ uint32_t lds[];
+    const int lane = threadIdx.x;
+    uint32_t* g = lds;                       // gsize words
+    uint32_t* dn = g + gsize;                // [m][64] prefix sums for one boson less right of the site
+    uint32_t* up = dn + m * HB_BLOCK;        // [m][64] and for one more
+    uint32_t* run = dn;                      // the wave's words, contiguous (dn and up are done with by then)
+    for (int a = lane; a < gsize; a += HB_BLOCK) g[a] = g_glob[a];
+    const int64_t q0 = static_cast<int64_t>(blockIdx.x) * HB_BLOCK, q = q0 + lane;
+    const bool valid = q < D;
+    const int64_t p = valid ? lex_of_pos[q] : 0;
+    // first word of this row: the tile's, the tile's earlier rows', the wave's earlier lanes'
+    const int64_t tq = q0 / HC_TILE;
+    int before = 0;
+    for (int64_t r = tq * HC_TILE + lane; r < q0; r += HB_BLOCK) before += cntg[r];
+    int inc = valid ? cntg[q] : 0;
+    const int cnt = inc;
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) before += __shfl_xor(before, o, 64);
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const int y = __shfl_up(inc, o, 64);
+        if (lane >= o) inc += y;
+    }
+    const int64_t wave0 = tile[tq] + before;
+    const int total = __shfl(inc, 63, 64), excl = inc - cnt;
+    if (valid) row_ptr[q] = static_cast<int32_t>(wave0 + excl);
+    if (q == D - 1) row_ptr[D] = static_cast<int32_t>(nnz);
+    __syncthreads();
+    PState<NW, BITS> s;
+    bh_unrank(p, m, n, g, s);
+    {
+        int R = n;
+        uint32_t d = 0, u = 0;
+#pragma unroll
+        for (int l = 0; l < PState<NW, BITS>::MAXM; ++l) {
+            if (l < m) {
+                dn[l * HB_BLOCK + lane] = d;
+                up[l * HB_BLOCK + lane] = u;
+                R -= s.get(l);
+                if (l < m - 1) {
+                    const uint32_t* gl = g + l * (n + 1);
+                    const uint32_t g0 = gl[R], gm = gl[max(R - 1, 0)], gp = gl[min(R + 1, n)];
+                    // R = 0 has no boson to lose, R = n none to gain: steps that no hop of this state uses
+                    d += R > 0 ? g0 - gm : 0u;
+                    u += R < n ? gp - g0 : 0u;
+                }
+            }
+        }
+    }
+    const uint32_t mask = (1u << cb) - 1u;
+    uint32_t w[P];
+#pragma unroll
+    for (int e = 0; e < P; ++e) {
+        w[e] = 0xffffffffu;
+        if (e < ed.E) {  // uniform
+            const int i = ed.ei[e], j = ed.ej[e], nj = s.get(j);
+            const uint32_t t = static_cast<uint32_t>(p) +
+                               (i < j ? dn[i * HB_BLOCK + lane] - dn[j * HB_BLOCK + lane] : up[i * HB_BLOCK + lane] - up[j * HB_BLOCK + lane]);
+            const uint32_t code = ed.cm[e] * static_cast<uint32_t>((s.get(i) + 1) * nj);
+            if (valid && nj >= 1) w[e] = (t << cb) | code;
+        }
+    }
+    if (pos_of_lex) {  // uniform: ranks to positions
+#pragma unroll
+        for (int e0 = 0; e0 < P; e0 += 8) {
+            uint32_t c[8];
+#pragma unroll
+            for (int e = e0; e < e0 + 8; ++e) c[e - e0] = static_cast<uint32_t>(pos_of_lex[w[e] == 0xffffffffu ? p : w[e] >> cb]);
+#pragma unroll
+            for (int e = e0; e < e0 + 8; ++e) w[e] = w[e] == 0xffffffffu ? w[e] : (c[e - e0] << cb) | (w[e] & mask);
+        }
+    }
+    sort_registers<P>(w);
+    __syncthreads();  // dn, up are read no more
+    double sum = 0.0;
+#pragma unroll
+    for (int a = 0; a < P; ++a) {
+        if (a < cnt) {
+            sum += table[w[a] & mask];
+            run[excl + a] = w[a];
+        }
+    }
+    __syncthreads();
+    for (int a = lane; a < total; a += HB_BLOCK) words[wave0 + a] = run[a];
     float v = 0.f;
     for (int i = 0; i < m; ++i) {
         const int ni = s.get(i);
         v += (flags & BH_CONV_REF_INTERACTION) ? static_cast<float>(ni * (ni + 1)) : static_cast<float>((ni * (ni - 1)) / 2);
     }
-    diag[q] = v;
+    if (valid) diag[q] = v;
+    // sums and V are not negative: their FP32 bit patterns order like the values
+    int mx = valid ? cnt : 0, ms = valid ? __float_as_int(static_cast<float>(sum) * 1.0001f) : 0;
+    int lo = valid ? __float_as_int(v) : 0x7f7fffff, hi = valid ? __float_as_int(v) : 0;
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) {
+        mx = max(mx, __shfl_xor(mx, o, 64));
+        ms = max(ms, __shfl_xor(ms, o, 64));
+        lo = min(lo, __shfl_xor(lo, o, 64));
+        hi = max(hi, __shfl_xor(hi, o, 64));
+    }
+    if (lane == 0) stats[blockIdx.x] = make_int4(mx, ms, lo, hi);
+}
+
+// the waves' statistics together (out starts at 0, 0, FLT_MAX, 0): one atomic a workgroup instead of four a row,
+// which took 983 us at D = 1,352,078
+__global__ void __launch_bounds__(256) k_ham_stats(const int4* __restrict__ stats, int64_t nb, int* __restrict__ out) {
+    __shared__ int4 red[4];
+    int4 a = make_int4(0, 0, 0x7f7fffff, 0);
+    for (int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; i < nb; i += static_cast<int64_t>(gridDim.x) * 256) {
+        const int4 x = stats[i];
+        a = make_int4(max(a.x, x.x), max(a.y, x.y), min(a.z, x.z), max(a.w, x.w));
+    }
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1)
+        a = make_int4(max(a.x, __shfl_xor(a.x, o, 64)), max(a.y, __shfl_xor(a.y, o, 64)), min(a.z, __shfl_xor(a.z, o, 64)),
+                      max(a.w, __shfl_xor(a.w, o, 64)));
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = a;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < 4; ++w)
+            a = make_int4(max(a.x, red[w].x), max(a.y, red[w].y), min(a.z, red[w].z), max(a.w, red[w].w));
+        atomicMax(out, a.x);
+        atomicMax(out + 1, a.y);
+        atomicMin(out + 2, a.z);
+        atomicMax(out + 3, a.w);
+    }
 }
 
 // Single-particle density matrix rho_ij = <phi| b_i^+ b_j |phi> (real phi), partial sums per workgroup.
@@ -182,20 +337,6 @@ __global__ void __launch_bounds__(256) k_spdm_sum(const double* __restrict__ par
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
     __syncthreads();
     if (threadIdx.x == 0) out[blockIdx.x] = (red[0] + red[1]) + (red[2] + red[3]);
-}
-
-// out[0]: longest row; out[1]: largest row sum of |T| (FP32 bits, non-negative); out[2], out[3]: min, max of V
-__global__ void k_row_stats(int64_t D, const int32_t* __restrict__ row_ptr, const uint32_t* __restrict__ words, int cb,
-                            const double* __restrict__ table, const float* __restrict__ diag, int* __restrict__ out) {
-    const int64_t r = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (r >= D) return;
-    const uint32_t mask = (1u << cb) - 1u;
-    double s = 0.0;
-    for (int32_t k = row_ptr[r]; k < row_ptr[r + 1]; ++k) s += table[words[k] & mask];
-    atomicMax(out, row_ptr[r + 1] - row_ptr[r]);
-    atomicMax(out + 1, __float_as_int(static_cast<float>(s) * 1.0001f));
-    atomicMin(out + 2, __float_as_int(diag[r]));
-    atomicMax(out + 3, __float_as_int(diag[r]));
 }
 
 #define BH_LAYOUT_DISPATCH(nw, bits, MACRO)             \
@@ -305,12 +446,7 @@ int bh_engine_choice(int B, const bh_ham* h) {
 static int free_ham(bh_ham* h) {
     bh_ctx* ctx = h->ctx;
     for (auto& kv : h->rowblocks) bh_dev_free(ctx, kv.second.first, static_cast<size_t>(kv.second.second + 1) * 8);
-    const size_t tab = (static_cast<size_t>(1) << h->code_bits);
-    bh_dev_free(ctx, h->row_ptr, static_cast<size_t>(h->D + 1) * sizeof(int32_t));
-    bh_dev_free(ctx, h->words, static_cast<size_t>(h->nnz + BH_WORDS_PAD) * sizeof(uint32_t));
-    bh_dev_free(ctx, h->diag, static_cast<size_t>(h->D) * sizeof(float));
-    bh_dev_free(ctx, h->table, tab * sizeof(double));
-    bh_dev_free(ctx, h->table32, tab * sizeof(float));
+    bh_dev_free(ctx, h->block, h->block_bytes);
     bh_dev_free(ctx, h->lex_of_pos, static_cast<size_t>(h->D) * sizeof(int32_t));
     delete h;
     return BH_OK;
@@ -373,6 +509,23 @@ int bh_hamiltonian_build(bh_ctx* ctx, const bh_basis* b, const int* nbr_off, con
     BH_HIP(ctx, hipSetDevice(ctx->device));
     hipStream_t s = ctx->stream;
 
+    // every directed bond (i, j) contributes an entry per state with a boson on j
+    const int64_t per_bond = n >= 1 ? bh_binom_host(m + n - 2, n - 1) : 0;
+    if (per_bond < 0 || per_bond > INT32_MAX || static_cast<int64_t>(E) * per_bond > INT32_MAX)
+        return bh_set_error(ctx, BH_ERANGE, "hamiltonian: number of entries exceeds the int32 index range");
+    const int64_t nnz = E * per_bond;
+    SiteDeg deg{};
+    for (int e = 0; e < E; ++e) deg.d[ej[e]] += 1;
+    // longest row possible: the busiest min(m, n) sites occupied
+    std::vector<int> dsort(deg.d, deg.d + m);
+    std::sort(dsort.rbegin(), dsort.rend());
+    int rowcap = 0;
+    for (int i = 0; i < std::min(m, n); ++i) rowcap += dsort[i];
+    rowcap = std::max(rowcap, 1);
+    const int gsize = (m > 1 ? m - 1 : 1) * (n + 1);
+    if ((static_cast<size_t>(gsize) + static_cast<size_t>(HB_BLOCK) * (E + 1)) * sizeof(uint32_t) > 64 * 1024) return bh_set_error(ctx, BH_ERANGE, "hamiltonian: rank table too large for LDS");
+    const size_t lds_bytes = (static_cast<size_t>(gsize) + static_cast<size_t>(HB_BLOCK) * std::max(rowcap, 2 * m)) * 4;
+
     std::unique_ptr<bh_ham> hp(new bh_ham());
     bh_ham* h = hp.get();
     h->ctx = ctx;
@@ -381,92 +534,96 @@ int bh_hamiltonian_build(bh_ctx* ctx, const bh_basis* b, const int* nbr_off, con
     h->code_bits = cb;
     h->flags = flags;
 
+    // one allocation: table, row pointers, diagonal, words
     const size_t tab = static_cast<size_t>(1) << cb;
-    std::vector<double> table(tab);
-    std::vector<float> table32(tab);
-    for (size_t c = 0; c < tab; ++c) {
-        table[c] = std::sqrt(static_cast<double>(c));
-        table32[c] = static_cast<float>(table[c]);
-    }
-    const int gsize = (m > 1 ? m - 1 : 1) * (n + 1);
-
-    DevArray<int8_t> dei, dej;
-    DevArray<uint32_t> dcm, words, dtab_dummy;
-    DevArray<int32_t> rownnz, row_ptr;
-    DevArray<float> diag, t32;
-    DevArray<double> t64;
-    DevArray<int> dmax;
-    BH_TRY(dei.alloc(ctx, std::max(E, 1)));
-    BH_TRY(dej.alloc(ctx, std::max(E, 1)));
-    BH_TRY(dcm.alloc(ctx, std::max(E, 1)));
-    BH_TRY(rownnz.alloc(ctx, static_cast<size_t>(D)));
-    BH_TRY(row_ptr.alloc(ctx, static_cast<size_t>(D + 1)));
-    BH_TRY(diag.alloc(ctx, static_cast<size_t>(D)));
-    BH_TRY(t64.alloc(ctx, tab));
-    BH_TRY(t32.alloc(ctx, tab));
-    BH_TRY(dmax.alloc(ctx, 4));
-    if (E) {
-        BH_HIP(ctx, hipMemcpyAsync(dei.p, ei.data(), E, hipMemcpyHostToDevice, s));
-        BH_HIP(ctx, hipMemcpyAsync(dej.p, ej.data(), E, hipMemcpyHostToDevice, s));
-        BH_HIP(ctx, hipMemcpyAsync(dcm.p, cm.data(), E * sizeof(uint32_t), hipMemcpyHostToDevice, s));
-    }
-    BH_HIP(ctx, hipMemcpyAsync(t64.p, table.data(), tab * sizeof(double), hipMemcpyHostToDevice, s));
-    BH_HIP(ctx, hipMemcpyAsync(t32.p, table32.data(), tab * sizeof(float), hipMemcpyHostToDevice, s));
-    EdgeArgs ed{E, dei.p, dej.p, dcm.p};
+    const size_t b_tab = BhScratch::size(tab * 8), b_rp = BhScratch::size(static_cast<size_t>(D + 1) * 4),
+                 b_dg = BhScratch::size(static_cast<size_t>(D) * 4), b_w = BhScratch::size(static_cast<size_t>(nnz + BH_WORDS_PAD) * 4);
+    DevArray<char> block;
+    BH_TRY(block.alloc(ctx, b_tab + b_rp + b_dg + b_w));
+    double* table = reinterpret_cast<double*>(block.p);
+    int32_t* row_ptr = reinterpret_cast<int32_t*>(block.p + b_tab);
+    float* diag = reinterpret_cast<float*>(block.p + b_tab + b_rp);
+    uint32_t* words = reinterpret_cast<uint32_t*>(block.p + b_tab + b_rp + b_dg);
+    // scratch: the small inputs (one copy), row counts, tile sums, the waves' statistics
+    const int64_t ntile = (D + HC_TILE - 1) / HC_TILE;
     const unsigned grid = static_cast<unsigned>((D + HB_BLOCK - 1) / HB_BLOCK);
+    const size_t b_in = 16 + static_cast<size_t>(std::max(E, 1)) * 4 + 2 * BhScratch::size(std::max(E, 1));
+    BhScratch sc;
+    BH_TRY(sc.open(ctx, BhScratch::size(b_in) + BhScratch::size(D) + BhScratch::size(ntile * 8) + BhScratch::size(static_cast<size_t>(grid) * 16)));
+    uint8_t* in = sc.take<uint8_t>(b_in);
+    uint8_t* cnt = sc.take<uint8_t>(D);
+    int64_t* tile = sc.take<int64_t>(ntile);
+    int4* wstats = sc.take<int4>(grid);
+    std::vector<uint8_t> hin(b_in, 0);  // row statistics' start values, code multipliers, targets, sources
+    int stats[4] = {0, 0, 0x7f7fffff, 0};
+    const size_t o_i = 16 + static_cast<size_t>(std::max(E, 1)) * 4, o_j = o_i + std::max(E, 1);
+    std::memcpy(hin.data(), stats, sizeof(stats));
+    for (int e = 0; e < E; ++e) {
+        std::memcpy(hin.data() + 16 + 4 * e, &cm[e], 4);
+        hin[o_i + e] = static_cast<uint8_t>(ei[e]);
+        hin[o_j + e] = static_cast<uint8_t>(ej[e]);
+    }
+    std::vector<double> htab(tab);
+    for (size_t c = 0; c < tab; ++c) htab[c] = std::sqrt(static_cast<double>(c));
+    BH_HIP(ctx, hipMemcpyAsync(in, hin.data(), o_j + std::max(E, 1), hipMemcpyHostToDevice, s));
+    BH_HIP(ctx, hipMemcpyAsync(table, htab.data(), tab * 8, hipMemcpyHostToDevice, s));
+    EdgeArgs ed{E, reinterpret_cast<int8_t*>(in + o_i), reinterpret_cast<int8_t*>(in + o_j), reinterpret_cast<uint32_t*>(in + 16)};
     {
         KTimer kt(ctx, "ham_count", s);
-#define LAUNCH_COUNT(NW_, BITS_)                                                                                   \
-    hipLaunchKernelGGL((k_ham_count<NW_, BITS_>), dim3(grid), dim3(HB_BLOCK), 0, s, D, m, n, b->rank_tab,         \
-                       b->lex_of_pos, ed, rownnz.p)
+#define LAUNCH_COUNT(NW_, BITS_)                                                                                        \
+    hipLaunchKernelGGL((k_ham_count<NW_, BITS_>), dim3(static_cast<unsigned>(ntile)), dim3(HC_BLOCK), gsize * 4, s, D,  \
+                       m, n, b->rank_tab, gsize, b->lex_of_pos, deg, cnt, tile)
         BH_LAYOUT_DISPATCH(b->nw, b->bits, LAUNCH_COUNT);
 #undef LAUNCH_COUNT
+        hipLaunchKernelGGL(k_scan_tiles, dim3(1), dim3(1024), 0, s, tile, ntile);
     }
     BH_HIP(ctx, hipGetLastError());
-    int64_t nnz = 0;
-    BH_TRY(bh_exclusive_scan_i32(ctx, rownnz.p, D, row_ptr.p, &nnz, s));
-    rownnz.reset();
-    BH_TRY(words.alloc(ctx, static_cast<size_t>(nnz + BH_WORDS_PAD)));
-    const size_t lds_bytes = (static_cast<size_t>(gsize) + static_cast<size_t>(HB_BLOCK) * (E + 1)) * sizeof(uint32_t);
-    if (lds_bytes > 64 * 1024) return bh_set_error(ctx, BH_ERANGE, "hamiltonian: rank table too large for LDS");
     {
         KTimer kt(ctx, "ham_fill", s);
-#define LAUNCH_FILL(NW_, BITS_)                                                                                    \
-    hipLaunchKernelGGL((k_ham_fill<NW_, BITS_>), dim3(grid), dim3(HB_BLOCK), lds_bytes, s, D, m, n, b->rank_tab,   \
-                       gsize, b->lex_of_pos, b->pos_of_lex, ed, cb, flags, row_ptr.p, words.p, diag.p)
+        const int32_t* pol = b->order == BH_ORDER_LEX ? nullptr : b->pos_of_lex;
+#define FILL(NW_, BITS_, P_)                                                                                            \
+    hipLaunchKernelGGL((k_ham_fill<NW_, BITS_, P_>), dim3(grid), dim3(HB_BLOCK), lds_bytes, s, D, m, n, b->rank_tab,    \
+                       gsize, b->lex_of_pos, pol, ed, cb, table, flags, cnt, tile, nnz, row_ptr, words, diag, wstats)
+#define LAUNCH_FILL(NW_, BITS_)            \
+    do {                                   \
+        if (E <= 8) FILL(NW_, BITS_, 8);   \
+        else if (E <= 16) FILL(NW_, BITS_, 16); \
+        else if (E <= 32) FILL(NW_, BITS_, 32); \
+        else if (E <= 64) FILL(NW_, BITS_, 64); \
+        else FILL(NW_, BITS_, 128);        \
+    } while (0)
         BH_LAYOUT_DISPATCH(b->nw, b->bits, LAUNCH_FILL);
 #undef LAUNCH_FILL
+#undef FILL
+        hipLaunchKernelGGL(k_ham_stats, dim3(std::min<unsigned>(64, (grid + 255) / 256)), dim3(256), 0, s, wstats,
+                           static_cast<int64_t>(grid), reinterpret_cast<int*>(in));
     }
     BH_HIP(ctx, hipGetLastError());
-    int stats[4] = {0, 0, 0x7f7fffff, 0};  // V >= 0, so FP32 bit patterns order like the values
-    BH_HIP(ctx, hipMemcpyAsync(dmax.p, stats, sizeof(stats), hipMemcpyHostToDevice, s));
-    hipLaunchKernelGGL(k_row_stats, dim3(static_cast<unsigned>((D + 255) / 256)), dim3(256), 0, s, D, row_ptr.p, words.p,
-                       cb, t64.p, diag.p, dmax.p);
-    BH_HIP(ctx, hipMemcpyAsync(stats, dmax.p, sizeof(stats), hipMemcpyDeviceToHost, s));
+    BH_HIP(ctx, hipMemcpyAsync(stats, in, sizeof(stats), hipMemcpyDeviceToHost, s));
+    DevArray<int32_t> lop;
+    if (bh_basis_lex_start(b)) {
+        BH_TRY(lop.alloc(ctx, static_cast<size_t>(D)));
+        BH_HIP(ctx, hipMemcpyAsync(lop.p, b->lex_of_pos, static_cast<size_t>(D) * sizeof(int32_t), hipMemcpyDeviceToDevice, s));
+    }
     BH_HIP(ctx, hipStreamSynchronize(s));
     auto as_f = [](int v) {
         float f;
         std::memcpy(&f, &v, 4);
         return static_cast<double>(f);
     };
-    DevArray<int32_t> lop;
-    if (bh_basis_lex_start(b)) {
-        BH_TRY(lop.alloc(ctx, static_cast<size_t>(D)));
-        BH_HIP(ctx, hipMemcpyAsync(lop.p, b->lex_of_pos, static_cast<size_t>(D) * sizeof(int32_t), hipMemcpyDeviceToDevice, s));
-        BH_HIP(ctx, hipStreamSynchronize(s));
-    }
     h->nnz = nnz;
     h->max_row = stats[0];
     h->tmax = as_f(stats[1]);
     h->vmin = as_f(stats[2]);
     h->vmax = as_f(stats[3]);
-    h->row_ptr = row_ptr.release();
-    h->words = words.release();
-    h->diag = diag.release();
-    h->table = t64.release();
-    h->table32 = t32.release();
+    h->row_ptr = row_ptr;
+    h->words = words;
+    h->diag = diag;
+    h->table = table;
+    h->block_bytes = block.bytes();
+    h->block = block.release();
     h->bytes = static_cast<size_t>(D + 1) * 4 + static_cast<size_t>(nnz ? nnz : 1) * 4 + static_cast<size_t>(D) * 4 +
-               tab * 12;
+               tab * 8;
     if (bh_basis_lex_start(b)) {
         h->lex_of_pos = lop.release();
         h->layout_id = b->layout_id;

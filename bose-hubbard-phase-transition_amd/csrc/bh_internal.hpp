@@ -32,6 +32,13 @@ struct bh_ctx {
     static constexpr int NWS = 8;
     void* ws[NWS] = {};
     size_t ws_bytes[NWS] = {};
+    // memory kept between calls, within the budget together with `used` and given up where that has no room: one freed block
+    // for the next allocation of about its size (bh_dev_free) and the builders' scratch (BhScratch)
+    void* spare = nullptr;
+    size_t spare_bytes = 0;
+    void* scratch = nullptr;
+    size_t scratch_bytes = 0;
+    bool scratch_busy = false;  // a builder is using it
     // start vector cached in workspace slot 3 for (r0_D, r0_seed), with the inverse norm of its copy in the
     // storage precision r0_mixed (1: FP32)
     int64_t r0_D = -1;
@@ -63,11 +70,42 @@ int bh_set_error(const bh_ctx* ctx, int code, const std::string& msg);
         if (rc_ != BH_OK) return rc_; \
     } while (0)
 
-// budgeted device allocation (bytes counted against ctx->budget)
+// budgeted device allocation (bytes counted against ctx->budget).  hipFree of a block from 32 MB up takes 0.22 ms (80 MB; 32 MB
+// and below 7 us), most of what building and dropping a sector costs beside its kernels, so the last such block
+// freed, up to BH_SPARE_MAX bytes, waits for the next allocation it fits (at most half as large again).  It is given up
+// when the budget or the device has no room beside it, and at the end of the context.  The device is
+// synchronised before a block is kept, as hipFree does.
+constexpr size_t BH_SPARE_MIN = size_t(32) << 20, BH_SPARE_MAX = size_t(256) << 20;
 int bh_dev_alloc(bh_ctx* ctx, void** p, size_t bytes);
 void bh_dev_free(bh_ctx* ctx, void* p, size_t bytes);
 // workspace slot of at least `bytes` (kept by the context until bh_ctx_destroy)
 int bh_ws_get(bh_ctx* ctx, int slot, size_t bytes, void** p);
+
+// Scratch of one builder call (basis, Hamiltonian, density matrix): up to BH_SCRATCH_KEEP bytes are kept by the context for
+// the next one, larger ones allocated and freed by the call.  bh_dev_alloc gives the kept bytes back when an
+// allocation does not fit beside them, bh_scratch_release at once.
+constexpr size_t BH_SCRATCH_KEEP = size_t(64) << 20;
+struct BhScratch {
+    bh_ctx* ctx = nullptr;
+    void* own = nullptr;
+    size_t own_bytes = 0;
+    char* base = nullptr;
+    size_t off = 0;
+    BhScratch() = default;
+    BhScratch(const BhScratch&) = delete;
+    BhScratch& operator=(const BhScratch&) = delete;
+    ~BhScratch();
+    int open(bh_ctx* c, size_t bytes);
+    static size_t size(size_t bytes) { return (bytes + 255) / 256 * 256; }
+    // the next `n` elements of the opened bytes
+    template <typename T>
+    T* take(size_t n) {
+        T* q = reinterpret_cast<T*>(base + off);
+        off += size(n * sizeof(T));
+        return q;
+    }
+};
+void bh_scratch_release(bh_ctx* ctx);
 
 // RAII device buffer
 template <typename T>
@@ -125,6 +163,8 @@ struct bh_basis {
     int32_t* lex_of_pos = nullptr;  // [D]
     int32_t* pos_of_lex = nullptr;  // [D]
     uint32_t* rank_tab = nullptr;   // [(m-1) * (n+1)] g[l][R] = C(R + m-l-2, m-l-1)
+    void* block = nullptr;          // the allocation the three arrays lie in
+    size_t block_bytes = 0;
     size_t bytes = 0;
     uint64_t layout_id = 0;         // new at every build and permutation (keys host caches of the layout)
 };
@@ -159,7 +199,8 @@ struct bh_ham {
     uint32_t* words = nullptr;    // [nnz + BH_WORDS_PAD] column << code_bits | code
     float* diag = nullptr;        // [D] V (exact small integers)
     double* table = nullptr;      // [1 << code_bits] sqrt(code), exact FP64
-    float* table32 = nullptr;     // [1 << code_bits] sqrt(code) rounded to FP32
+    void* block = nullptr;        // the allocation row_ptr, words, diag and table lie in
+    size_t block_bytes = 0;
     bool prepared64 = false;      // bh_ham_prepare or bh_spmv has been called for FP64 (bh_spmv_noalloc asks for it)
     size_t bytes = 0;
     // spectral bounds: V in [vmin, vmax]; the largest row sum of |T| (Gershgorin radius of T)
@@ -220,19 +261,30 @@ struct PState {
 
 // lexicographic unranking, descending order (src/hamiltonian.cpp:60-85):
 // rank(s) = sum_{l=0}^{m-2} g[l][Rem_l],  Rem_l = n - sum_{l'<=l} s_l',  g[l][R] = C(R + m-l-2, m-l-1)
+// The remainder after a site is the largest K with g[K] <= rest (g ascends; K <= R since rest < g[R + 1]): a bisection of
+// ceil(log2(n + 1)) steps, the same number for every lane, on a table the caller has put in LDS (keys of D = 1,352,078
+// states: 70 us searching upwards in global memory, 28 us so, 40 us comparing every K against scalar loads).
 template <int NW, int BITS>
-__device__ __forceinline__ void bh_unrank(int64_t r, int m, int n, const uint32_t* __restrict__ g,
+__device__ __forceinline__ void bh_unrank(int64_t r, int m, int n, const uint32_t* g,
                                           PState<NW, BITS>& s) {
     s.clear();
     int R = n;
-    int64_t rr = r;
+    uint32_t rr = static_cast<uint32_t>(r);  // ranks are below D < 2^31
+    const int top = n > 0 ? 1 << (31 - __clz(n)) : 0;
 #pragma unroll
     for (int i = 0; i < PState<NW, BITS>::MAXM - 1; ++i) {
         if (i < m - 1) {
             const uint32_t* gi = g + static_cast<size_t>(i) * (n + 1);
             int K = 0;
-            while (K < R && static_cast<int64_t>(gi[K + 1]) <= rr) ++K;
-            rr -= gi[K];
+            uint32_t gk = 0;  // g[0] = 0
+            for (int b = top; b > 0; b >>= 1) {
+                const int k = K + b;
+                const uint32_t x = gi[min(k, n)];
+                const bool c = k <= n && x <= rr;
+                K = c ? k : K;
+                gk = c ? x : gk;
+            }
+            rr -= gk;
             s.put(i, R - K);
             R = K;
         }
@@ -241,6 +293,12 @@ __device__ __forceinline__ void bh_unrank(int64_t r, int m, int n, const uint32_
 #pragma unroll
     for (int i = 0; i < PState<NW, BITS>::MAXM; ++i)
         if (i == m - 1) s.put(i, R);
+}
+
+// the rank table (gsize words) into LDS, by the whole workgroup
+__device__ __forceinline__ void bh_stage_table(const uint32_t* __restrict__ g, int gsize, uint32_t* lds) {
+    for (int a = threadIdx.x; a < gsize; a += blockDim.x) lds[a] = g[a];
+    __syncthreads();
 }
 
 // ---- host helpers ----------------------------------------------------------------------------------

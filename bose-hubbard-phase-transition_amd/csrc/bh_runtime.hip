@@ -15,14 +15,71 @@ int bh_set_error(const bh_ctx* ctx, int code, const std::string& msg) {
     return code;
 }
 
+static void spare_release(bh_ctx* ctx) {
+    if (!ctx->spare) return;
+    (void)hipFree(ctx->spare);
+    ctx->spare = nullptr;
+    ctx->spare_bytes = 0;
+}
+
+void bh_scratch_release(bh_ctx* ctx) {
+    if (ctx->scratch_busy || !ctx->scratch) return;
+    (void)hipFree(ctx->scratch);
+    ctx->scratch = nullptr;
+    ctx->scratch_bytes = 0;
+}
+
+int BhScratch::open(bh_ctx* c, size_t bytes) {
+    ctx = c;
+    off = 0;
+    if (bytes <= BH_SCRATCH_KEEP && !c->scratch_busy) {
+        if (c->scratch_bytes < bytes) {
+            bh_scratch_release(c);
+            void* q = nullptr;
+            BH_TRY(bh_dev_alloc(c, &q, bytes));
+            c->used -= bytes;
+            c->scratch = q;
+            c->scratch_bytes = bytes;
+        }
+        c->scratch_busy = true;
+        base = static_cast<char*>(c->scratch);
+        return BH_OK;
+    }
+    BH_TRY(bh_dev_alloc(c, &own, bytes));
+    own_bytes = bytes;
+    base = static_cast<char*>(own);
+    return BH_OK;
+}
+
+BhScratch::~BhScratch() {
+    if (!base) return;
+    if (own) bh_dev_free(ctx, own, own_bytes);
+    else ctx->scratch_busy = false;
+}
+
 int bh_dev_alloc(bh_ctx* ctx, void** p, size_t bytes) {
     *p = nullptr;
-    if (ctx->used + bytes > ctx->budget)
+    if (ctx->spare && ctx->spare_bytes >= bytes && ctx->spare_bytes - bytes <= bytes / 2 && ctx->used + ctx->spare_bytes + ctx->scratch_bytes <= ctx->budget) {
+        *p = ctx->spare;
+        ctx->spare = nullptr;
+        ctx->spare_bytes = 0;
+        ctx->used += bytes;
+        return BH_OK;
+    }
+    if (ctx->used + ctx->spare_bytes + ctx->scratch_bytes + bytes > ctx->budget) spare_release(ctx);
+    if (ctx->used + ctx->scratch_bytes + bytes > ctx->budget) bh_scratch_release(ctx);
+    if (ctx->used + ctx->scratch_bytes + bytes > ctx->budget)
         return bh_set_error(ctx, BH_EBUDGET,
                             "HBM budget exceeded: need " + std::to_string(bytes) + " B, used " +
-                                std::to_string(ctx->used) + " of " + std::to_string(ctx->budget));
+                                std::to_string(ctx->used + ctx->scratch_bytes) + " of " + std::to_string(ctx->budget));
     const auto t0 = std::chrono::steady_clock::now();
     hipError_t e = hipMalloc(p, bytes);
+    if (e != hipSuccess && (ctx->spare || (ctx->scratch && !ctx->scratch_busy))) {
+        (void)hipGetLastError();
+        spare_release(ctx);
+        bh_scratch_release(ctx);
+        e = hipMalloc(p, bytes);
+    }
     ctx->n_alloc += 1;
     ctx->alloc_ms += std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
     if (e != hipSuccess) {
@@ -36,7 +93,13 @@ int bh_dev_alloc(bh_ctx* ctx, void** p, size_t bytes) {
 void bh_dev_free(bh_ctx* ctx, void* p, size_t bytes) {
     if (!p) return;
     const auto t0 = std::chrono::steady_clock::now();
-    (void)hipFree(p);
+    if (bytes >= BH_SPARE_MIN && bytes <= BH_SPARE_MAX && hipDeviceSynchronize() == hipSuccess) {
+        spare_release(ctx);
+        ctx->spare = p;
+        ctx->spare_bytes = bytes;
+    } else {
+        (void)hipFree(p);
+    }
     ctx->n_free += 1;
     ctx->free_ms += std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
     ctx->used = ctx->used >= bytes ? ctx->used - bytes : 0;
@@ -181,6 +244,8 @@ int bh_ctx_destroy(bh_ctx* ctx) {
         (void)hipStreamSynchronize(ctx->stream);
         bh_ktimers_flush(ctx);
         for (int i = 0; i < bh_ctx::NWS; ++i) bh_dev_free(ctx, ctx->ws[i], ctx->ws_bytes[i]);
+        spare_release(ctx);
+        bh_scratch_release(ctx);
         (void)hipStreamDestroy(ctx->stream);
     }
     delete ctx;
