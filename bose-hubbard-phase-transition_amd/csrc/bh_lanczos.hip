@@ -2274,16 +2274,12 @@ class LzEngine final : public LzEngineBase {
                 BH_HIP(ctx, hipStreamSynchronize(s));
             }
             // exact FP64 operator on each candidate (packed words, FP64 table, FP64 vectors)
-            DevArray<double> dJ, dU;
-            BH_TRY(dJ.alloc(ctx, B));
-            BH_TRY(dU.alloc(ctx, B));
-            BH_HIP(ctx, hipMemcpyAsync(dJ.p, Jb.data(), B * 8, hipMemcpyHostToDevice, s));
-            BH_HIP(ctx, hipMemcpyAsync(dU.p, Ub.data(), B * 8, hipMemcpyHostToDevice, s));
+            const SpmvCoef coef = bh_spmv_coef(Jb.data(), Ub.data(), B);
             for (int i = 0; i < nvf; ++i) {
                 KTimer kt(ctx, "lanczos_finish_spmv", s);
                 SpmvArgs<double> sa{D, h->row_ptr, h->words, h->diag, h->table, h->code_bits,
-                                    dJ.p, dU.p, Yfp + static_cast<int64_t>(i) * vs, HYp + static_cast<int64_t>(i) * vs, 1};
-                BH_TRY(bh_apply(ctx, h, sa, BH_KEY_FINISH, B, s));
+                                    nullptr, nullptr, Yfp + static_cast<int64_t>(i) * vs, HYp + static_cast<int64_t>(i) * vs, 1};
+                BH_TRY(bh_apply(ctx, h, sa, coef, BH_KEY_FINISH, B, s));
             }
             BH_HIP(ctx, hipGetLastError());
             BH_TRY(rayleigh_ritz(lanes, nvf, nt, Yfp, HYp));
@@ -2500,18 +2496,17 @@ class LzEngine final : public LzEngineBase {
         for (auto& v : th0)
             if (!std::isfinite(v)) v = 0.0;
         for (int b = 0; b < B; ++b) dl[b] = LZ_REFINE_CLAMP * std::fmax(std::fmax(std::fabs(Ub[b]), std::fabs(Jb[b])), 1e-300);
-        DevArray<double> dth, ddl, dU, dJ, df;
+        DevArray<double> dth, ddl, dU, df;
+        const SpmvCoef coef = bh_spmv_coef(Jb.data(), Ub.data(), B);
         DevArray<int> don;
         BH_TRY(dth.alloc(ctx, th0.size()));
         BH_TRY(ddl.alloc(ctx, B));
         BH_TRY(dU.alloc(ctx, B));
-        BH_TRY(dJ.alloc(ctx, B));
         BH_TRY(df.alloc(ctx, static_cast<size_t>(np) * B));
         BH_TRY(don.alloc(ctx, B));
         BH_HIP(ctx, hipMemcpyAsync(dth.p, th0.data(), th0.size() * 8, hipMemcpyHostToDevice, s));
         BH_HIP(ctx, hipMemcpyAsync(ddl.p, dl.data(), B * 8, hipMemcpyHostToDevice, s));
         BH_HIP(ctx, hipMemcpyAsync(dU.p, Ub.data(), B * 8, hipMemcpyHostToDevice, s));
-        BH_HIP(ctx, hipMemcpyAsync(dJ.p, Jb.data(), B * 8, hipMemcpyHostToDevice, s));
         BH_HIP(ctx, hipMemcpyAsync(don.p, on.data(), B * sizeof(int), hipMemcpyHostToDevice, s));
         {
             KTimer kt(ctx, "lanczos_refine", s);
@@ -2540,8 +2535,8 @@ class LzEngine final : public LzEngineBase {
         for (int i = 0; i < np; ++i) {
             KTimer kt(ctx, "lanczos_finish_spmv", s);
             SpmvArgs<double> sa{D, h->row_ptr, h->words, h->diag, h->table, h->code_bits,
-                                dJ.p, dU.p, Tp + static_cast<int64_t>(i) * vs, HTp + static_cast<int64_t>(i) * vs, 1};
-            BH_TRY(bh_apply(ctx, h, sa, BH_KEY_FINISH, B, s));
+                                nullptr, nullptr, Tp + static_cast<int64_t>(i) * vs, HTp + static_cast<int64_t>(i) * vs, 1};
+            BH_TRY(bh_apply(ctx, h, sa, coef, BH_KEY_FINISH, B, s));
         }
         BH_HIP(ctx, hipGetLastError());
         std::vector<int> lr, n2(B, 0);

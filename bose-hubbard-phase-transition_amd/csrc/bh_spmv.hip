@@ -14,18 +14,33 @@
 #include "bh_kernels.hpp"
 #include "bh_spmv.hpp"
 
-template <int WG>
-__device__ __forceinline__ void spmv_table(const double* __restrict__ table, int cb, double* tab) {
-    for (int i = threadIdx.x; i < (1 << cb); i += WG) tab[i] = table[i];
+// the value table and the lanes' coefficients in LDS
+template <typename XT, int B>
+__device__ __forceinline__ void spmv_setup(const SpmvArgs<XT>& a, const SpmvCoef& c, double* tab, double* cJ, double* cU) {
+    for (int i = threadIdx.x; i < (1 << a.cb); i += BH_WG) tab[i] = a.table[i];
+    if (threadIdx.x < B) {
+        cJ[threadIdx.x] = a.J ? a.J[threadIdx.x] : c.J[threadIdx.x];
+        cU[threadIdx.x] = a.J ? a.U[threadIdx.x] : c.U[threadIdx.x];
+    }
     __syncthreads();
 }
 
+SpmvCoef bh_spmv_coef(const double* J, const double* U, int B) {
+    SpmvCoef c;
+    for (int b = 0; b < 64; ++b) {
+        c.J[b] = b < B ? J[b] : 0.0;
+        c.U[b] = b < B ? U[b] : 0.0;
+    }
+    return c;
+}
+
 template <typename XT, int B, int G>
-__global__ void __launch_bounds__(BH_WG) k_spmv(SpmvArgs<XT> a) {
+__global__ void __launch_bounds__(BH_WG) k_spmv(SpmvArgs<XT> a, SpmvCoef c) {
     constexpr int GB = G * B;
     constexpr int SLOTS = BH_WG / GB;
     extern __shared__ double tab[];  // (1 << cb) entries
-    spmv_table<BH_WG>(a.table, a.cb, tab);
+    __shared__ double cJ[B], cU[B];
+    spmv_setup<XT, B>(a, c, tab, cJ, cU);
     const int lane = threadIdx.x;
     const int slot = lane / GB;
     const int g = (lane % GB) / B;
@@ -39,20 +54,21 @@ __global__ void __launch_bounds__(BH_WG) k_spmv(SpmvArgs<XT> a) {
     acc = bh_group_sum<B, G>(acc);
     if (g == 0 && r < a.D) {
         const double xr = to_d(a.x[r * B + b]);
-        a.y[r * B + b] = static_cast<XT>(a.J[b] * -acc + a.U[b] * static_cast<double>(a.diag[r]) * xr);
+        a.y[r * B + b] = static_cast<XT>(cJ[b] * -acc + cU[b] * static_cast<double>(a.diag[r]) * xr);
     }
 }
 
 template <typename XT, int B>
-__global__ void __launch_bounds__(BH_WG) k_spmv_rb(SpmvArgs<XT> a, const int32_t* __restrict__ rb, int64_t nblocks) {
+__global__ void __launch_bounds__(BH_WG) k_spmv_rb(SpmvArgs<XT> a, SpmvCoef c, const int32_t* __restrict__ rb, int64_t nblocks) {
     extern __shared__ double smem[];
     double* tab = smem;  // (1 << cb) entries
     double* prod = smem + (1 << a.cb);
-    spmv_table<BH_WG>(a.table, a.cb, tab);
+    __shared__ double cJ[B], cU[B];
+    spmv_setup<XT, B>(a, c, tab, cJ, cU);
     const int64_t t = a.xcd ? bh_xcd_tile(blockIdx.x, gridDim.x) : blockIdx.x;
     auto epi = [&](int64_t r, int bb, const double (&sum)[1]) {
         const double d = static_cast<double>(a.diag[r]);
-        a.y[r * B + bb] = static_cast<XT>(a.J[bb] * -sum[0] + a.U[bb] * d * to_d(a.x[r * B + bb]));
+        a.y[r * B + bb] = static_cast<XT>(cJ[bb] * -sum[0] + cU[bb] * d * to_d(a.x[r * B + bb]));
     };
     bh_rowblock_run<XT, B, BH_WG>(t, t + 1, rb, a.row_ptr, a.words, tab, a.cb, a.x, prod, epi);
 }
@@ -61,36 +77,39 @@ __global__ void __launch_bounds__(BH_WG) k_spmv_rb(SpmvArgs<XT> a, const int32_t
 template <typename XT, int B, int V>
 struct SpmvEpi {
     const SpmvArgs<XT>& a;
+    const double *cJ, *cU;
     __device__ __forceinline__ void operator()(int64_t r, int b0, const double (&acc)[V]) const {
         const double d = static_cast<double>(a.diag[r]);
         const BhVec<XT, V> xv = bh_vload<V>(a.x + r * B + b0);
         BhVec<XT, V> yv;
 #pragma unroll
         for (int v = 0; v < V; ++v)
-            yv.v[v] = static_cast<XT>(a.J[b0 + v] * -acc[v] + a.U[b0 + v] * d * to_d(xv.v[v]));
+            yv.v[v] = static_cast<XT>(cJ[b0 + v] * -acc[v] + cU[b0 + v] * d * to_d(xv.v[v]));
         *reinterpret_cast<BhVec<XT, V>*>(a.y + r * B + b0) = yv;
     }
 };
 
 template <typename XT, int B, int V>
-__global__ void __launch_bounds__(BH_WG) k_spmv_rl(SpmvArgs<XT> a, int64_t rows_per_wg) {
+__global__ void __launch_bounds__(BH_WG) k_spmv_rl(SpmvArgs<XT> a, SpmvCoef c, int64_t rows_per_wg) {
     extern __shared__ double tab[];
-    spmv_table<BH_WG>(a.table, a.cb, tab);
+    __shared__ double cJ[B], cU[B];
+    spmv_setup<XT, B>(a, c, tab, cJ, cU);
     const int64_t t = a.xcd ? bh_xcd_tile(blockIdx.x, gridDim.x) : blockIdx.x;
     const int64_t r0 = min(t * rows_per_wg, a.D), r1 = min(r0 + rows_per_wg, a.D);
-    SpmvEpi<XT, B, V> epi{a};
+    SpmvEpi<XT, B, V> epi{a, cJ, cU};
     bh_rowlane_run<XT, B, V, BH_WG, 4>(r0, r1, a.row_ptr, a.words, tab, a.cb, a.x, epi);
 }
 
 // one thread per row (V = B): the words of a wave's 64 rows go through LDS
 template <typename XT, int V>
-__global__ void __launch_bounds__(BH_WG) k_spmv_rt(SpmvArgs<XT> a, int64_t rows_per_wg, int cap) {
+__global__ void __launch_bounds__(BH_WG) k_spmv_rt(SpmvArgs<XT> a, SpmvCoef c, int64_t rows_per_wg, int cap) {
     extern __shared__ __align__(16) double smem[];
     double* tab = smem;
-    spmv_table<BH_WG>(a.table, a.cb, tab);
+    __shared__ double cJ[V], cU[V];
+    spmv_setup<XT, V>(a, c, tab, cJ, cU);
     const int64_t t = a.xcd ? bh_xcd_tile(blockIdx.x, gridDim.x) : blockIdx.x;
     const int64_t r0 = min(t * rows_per_wg, a.D), r1 = min(r0 + rows_per_wg, a.D);
-    SpmvEpi<XT, V, V> epi{a};
+    SpmvEpi<XT, V, V> epi{a, cJ, cU};
     bh_rowtile_run<XT, V, BH_WG, (V == 1 ? 8 : 4)>(r0, r1, a.row_ptr, a.words, tab, a.cb, a.x,
                                                    reinterpret_cast<uint32_t*>(smem + (1 << a.cb)), cap, epi);
 }
@@ -102,7 +121,7 @@ int bh_tile_cap(const bh_ham* h) {
 
 // row-lane engine with V vectors per thread (V * sizeof(XT) <= 16 bytes, V <= B); one thread per row: row tiles
 template <typename XT>
-static void launch_spmv_rl(const bh_ham* h, const SpmvArgs<XT>& a, int B, int V, hipStream_t s) {
+static void launch_spmv_rl(const bh_ham* h, const SpmvArgs<XT>& a, const SpmvCoef& c, int B, int V, hipStream_t s) {
     const size_t shm = (static_cast<size_t>(1) << a.cb) * sizeof(double);
     // up to four passes of BH_WG V / B rows per workgroup, fewer while that leaves under 1024 workgroups (four per CU)
     const int64_t pass = static_cast<int64_t>(BH_WG) * V / B;
@@ -111,15 +130,15 @@ static void launch_spmv_rl(const bh_ham* h, const SpmvArgs<XT>& a, int B, int V,
     if (B == V) {
         const int cap = bh_tile_cap(h);
         const size_t sht = shm + static_cast<size_t>(BH_WG / 64) * cap * sizeof(uint32_t);
-        if (V == 1) hipLaunchKernelGGL((k_spmv_rt<XT, 1>), dim3(grid), dim3(BH_WG), sht, s, a, rows_per_wg, cap);
-        else if (V == 2) hipLaunchKernelGGL((k_spmv_rt<XT, 2>), dim3(grid), dim3(BH_WG), sht, s, a, rows_per_wg, cap);
+        if (V == 1) hipLaunchKernelGGL((k_spmv_rt<XT, 1>), dim3(grid), dim3(BH_WG), sht, s, a, c, rows_per_wg, cap);
+        else if (V == 2) hipLaunchKernelGGL((k_spmv_rt<XT, 2>), dim3(grid), dim3(BH_WG), sht, s, a, c, rows_per_wg, cap);
         if constexpr (sizeof(XT) == 4)
-            if (V == 4) hipLaunchKernelGGL((k_spmv_rt<XT, 4>), dim3(grid), dim3(BH_WG), sht, s, a, rows_per_wg, cap);
+            if (V == 4) hipLaunchKernelGGL((k_spmv_rt<XT, 4>), dim3(grid), dim3(BH_WG), sht, s, a, c, rows_per_wg, cap);
         return;
     }
 #define L(BB, VV)                                                                                             \
     if (B == BB && V == VV) {                                                                                 \
-        hipLaunchKernelGGL((k_spmv_rl<XT, BB, VV>), dim3(grid), dim3(BH_WG), shm, s, a, rows_per_wg);         \
+        hipLaunchKernelGGL((k_spmv_rl<XT, BB, VV>), dim3(grid), dim3(BH_WG), shm, s, a, c, rows_per_wg);       \
         return;                                                                                               \
     }
     L(2, 1) L(4, 1) L(8, 1) L(16, 1) L(32, 1) L(64, 1)
@@ -131,12 +150,12 @@ static void launch_spmv_rl(const bh_ham* h, const SpmvArgs<XT>& a, int B, int V,
 }
 
 template <typename XT>
-static void launch_spmv_rb(const SpmvArgs<XT>& a, int B, const int32_t* rb, int64_t nb, hipStream_t s) {
+static void launch_spmv_rb(const SpmvArgs<XT>& a, const SpmvCoef& c, int B, const int32_t* rb, int64_t nb, hipStream_t s) {
     const size_t shm = ((static_cast<size_t>(1) << a.cb) + BH_STAGE_PRODUCTS) * sizeof(double);
     const unsigned grid = static_cast<unsigned>(nb);
 #define L(BB)                                                                                       \
     if (B == BB) {                                                                                  \
-        hipLaunchKernelGGL((k_spmv_rb<XT, BB>), dim3(grid), dim3(BH_WG), shm, s, a, rb, nb);        \
+        hipLaunchKernelGGL((k_spmv_rb<XT, BB>), dim3(grid), dim3(BH_WG), shm, s, a, c, rb, nb);     \
         return;                                                                                     \
     }
     L(1) L(2) L(4) L(8) L(16) L(32) L(64)
@@ -144,14 +163,14 @@ static void launch_spmv_rb(const SpmvArgs<XT>& a, int B, const int32_t* rb, int6
 }
 
 template <typename XT>
-static void launch_spmv_g(const SpmvArgs<XT>& a, int B, int G, hipStream_t s) {
+static void launch_spmv_g(const SpmvArgs<XT>& a, const SpmvCoef& c, int B, int G, hipStream_t s) {
     const int GB = G * B;
     const int64_t slots = BH_WG / GB;
     const unsigned grid = static_cast<unsigned>((a.D + slots - 1) / slots);
     const size_t shm = (static_cast<size_t>(1) << a.cb) * sizeof(double);
 #define L(BB, GG)                                                                          \
     if (B == BB && G == GG) {                                                              \
-        hipLaunchKernelGGL((k_spmv<XT, BB, GG>), dim3(grid), dim3(BH_WG), shm, s, a);      \
+        hipLaunchKernelGGL((k_spmv<XT, BB, GG>), dim3(grid), dim3(BH_WG), shm, s, a, c);   \
         return;                                                                            \
     }
     L(1, 1) L(1, 2) L(1, 4) L(1, 8) L(1, 16) L(1, 32) L(1, 64)
@@ -167,16 +186,16 @@ static void launch_spmv_g(const SpmvArgs<XT>& a, int B, int G, hipStream_t s) {
 // SpMV variants: 0 = LDS-staged row blocks; V = 1, 2, 4 = V vectors per thread, B / V threads per row (64 V / B
 // rows per wavefront); 100 + G = G lanes per row (64 / (G B) rows per wavefront)
 template <typename XT>
-static int spmv_launch(bh_ham* h, int var, const SpmvArgs<XT>& a, int B, hipStream_t s) {
+static int spmv_launch(bh_ham* h, int var, const SpmvArgs<XT>& a, const SpmvCoef& c, int B, hipStream_t s) {
     if (var == 0) {
         const int32_t* rb = nullptr;
         int64_t nb = 0;
         BH_TRY(bh_ham_rowblocks(h, B, &rb, &nb));
-        launch_spmv_rb(a, B, rb, nb, s);
+        launch_spmv_rb(a, c, B, rb, nb, s);
     } else if (var >= 100) {
-        launch_spmv_g(a, B, var - 100, s);
+        launch_spmv_g(a, c, B, var - 100, s);
     } else {
-        launch_spmv_rl(h, a, B, var, s);
+        launch_spmv_rl(h, a, c, B, var, s);
     }
     return BH_OK;
 }
@@ -186,17 +205,17 @@ static int spmv_launch(bh_ham* h, int var, const SpmvArgs<XT>& a, int B, hipStre
 // timed with HIP events over a warm-up and three applications to the caller's own x and y (y = H x is
 // idempotent), and the fastest is kept in the handle.  Under stream capture the default variant is used.
 template <typename XT>
-static int apply_t(bh_ctx* ctx, bh_ham* h, const SpmvArgs<XT>& a, int prec, int B, hipStream_t s) {
+static int apply_t(bh_ctx* ctx, bh_ham* h, const SpmvArgs<XT>& a, const SpmvCoef& c, int prec, int B, hipStream_t s) {
     const int key = bh_tune_key(1, prec, B);
     std::lock_guard<std::recursive_mutex> lk(ctx->mu);
     auto it = h->tuned.find(key);
-    if (it != h->tuned.end()) return spmv_launch(h, it->second.variant, a, B, s);
+    if (it != h->tuned.end()) return spmv_launch(h, it->second.variant, a, c, B, s);
     const int eng = bh_engine_choice(B, h);
     BhTuned t;
     t.variant = eng == 2 ? 1 : (eng == 1 ? 0 : 100 + bh_pick_lanes(h, B));
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     BH_HIP(ctx, hipStreamIsCapturing(s, &cs));
-    if (cs != hipStreamCaptureStatusNone) return spmv_launch(h, t.variant, a, B, s);
+    if (cs != hipStreamCaptureStatusNone) return spmv_launch(h, t.variant, a, c, B, s);
     if (bh_tune_enabled() && bh_engine_env() < 0) {
         std::vector<int> cand;
         if (static_cast<int64_t>(h->max_row) * B <= BH_STAGE_PRODUCTS_HOST) cand.push_back(0);
@@ -210,9 +229,9 @@ static int apply_t(bh_ctx* ctx, bh_ham* h, const SpmvArgs<XT>& a, int prec, int 
         BH_HIP(ctx, hipEventCreate(&e1));
         double best = 0.0;
         for (int var : cand) {
-            BH_TRY(spmv_launch(h, var, a, B, s));
+            BH_TRY(spmv_launch(h, var, a, c, B, s));
             BH_HIP(ctx, hipEventRecord(e0, s));
-            for (int r = 0; r < 3; ++r) BH_TRY(spmv_launch(h, var, a, B, s));
+            for (int r = 0; r < 3; ++r) BH_TRY(spmv_launch(h, var, a, c, B, s));
             BH_HIP(ctx, hipEventRecord(e1, s));
             BH_HIP(ctx, hipEventSynchronize(e1));
             float ms = 0.f;
@@ -228,14 +247,14 @@ static int apply_t(bh_ctx* ctx, bh_ham* h, const SpmvArgs<XT>& a, int prec, int 
         (void)hipEventDestroy(e1);
     }
     h->tuned[key] = t;
-    return spmv_launch(h, t.variant, a, B, s);
+    return spmv_launch(h, t.variant, a, c, B, s);
 }
 
-int bh_apply(bh_ctx* ctx, bh_ham* h, const SpmvArgs<double>& a, int key, int B, hipStream_t s) {
-    return apply_t(ctx, h, a, key, B, s);
+int bh_apply(bh_ctx* ctx, bh_ham* h, const SpmvArgs<double>& a, const SpmvCoef& c, int key, int B, hipStream_t s) {
+    return apply_t(ctx, h, a, c, key, B, s);
 }
-int bh_apply(bh_ctx* ctx, bh_ham* h, const SpmvArgs<float>& a, int key, int B, hipStream_t s) {
-    return apply_t(ctx, h, a, key, B, s);
+int bh_apply(bh_ctx* ctx, bh_ham* h, const SpmvArgs<float>& a, const SpmvCoef& c, int key, int B, hipStream_t s) {
+    return apply_t(ctx, h, a, c, key, B, s);
 }
 
 int bh_pick_lanes(const bh_ham* h, int B) {
@@ -255,11 +274,10 @@ double bh_spmv_bytes(const bh_ham* h, int prec, int B) {
 int bh_is_pow2_le64(int B) { return B >= 1 && B <= 64 && (B & (B - 1)) == 0; }
 
 // ---- the SpMV entry point that allocates nothing -------------------------------------------------------------
-// bh_spmv stages the per-lane coefficients J_b, U_b in two small device arrays it allocates per call.  Callers that
-// cannot allocate (code under HIP graph capture, tight serving loops) use bh_spmv_noalloc: the coefficients go to
-// this file-scope array instead, whose device address is looked up once per device with hipGetSymbolAddress (the
-// array's name in host code is a host-side stand-in, never a device address).  Every call on a device shares
-// that device's copy, so calls that overlap on one device race.
+// The coefficients go with the launch.  Under stream capture they are staged in this file-scope array instead, whose device
+// address is looked up once per device with hipGetSymbolAddress (the array's name in host code is a host-side
+// stand-in, never a device address), by copies that each replay repeats from the caller's arrays.  Every captured
+// call on a device shares that device's copy, so graphs that overlap on one device race.
 namespace {
 constexpr int SPMV_SCRATCH_LANES = 64;  // the largest batch width of the SpMV kernels
 static __device__ __align__(256) double scratch[2 * SPMV_SCRATCH_LANES];
@@ -295,10 +313,18 @@ int bh_spmv_noalloc(bh_ctx* ctx, bh_ham* h, int prec, int B, const double* J, co
     if (prec == BH_PREC_FP64 && !h->prepared64)
         return bh_set_error(ctx, BH_EINVAL, "spmv_noalloc: handle not prepared for FP64 (bh_ham_prepare first)");
     hipStream_t s = stream ? static_cast<hipStream_t>(stream) : ctx->stream;
-    double* sc = nullptr;
-    BH_TRY(scratch_ptr(ctx, &sc));
-    BH_HIP(ctx, hipMemcpyAsync(sc, J, B * sizeof(double), hipMemcpyHostToDevice, s));
-    BH_HIP(ctx, hipMemcpyAsync(sc + SPMV_SCRATCH_LANES, U, B * sizeof(double), hipMemcpyHostToDevice, s));
+    // under capture the coefficients are staged in the device array by copies that a replay repeats from the caller's
+    // J and U; otherwise they go with the launch
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    BH_HIP(ctx, hipStreamIsCapturing(s, &cs));
+    const SpmvCoef c = bh_spmv_coef(J, U, B);
+    double *dJ = nullptr, *dU = nullptr;
+    if (cs != hipStreamCaptureStatusNone) {
+        BH_TRY(scratch_ptr(ctx, &dJ));
+        dU = dJ + SPMV_SCRATCH_LANES;
+        BH_HIP(ctx, hipMemcpyAsync(dJ, J, B * sizeof(double), hipMemcpyHostToDevice, s));
+        BH_HIP(ctx, hipMemcpyAsync(dU, U, B * sizeof(double), hipMemcpyHostToDevice, s));
+    }
     // the variant the autotuner chose for this sector (no tuning here: it times with events), else the default
     // bh_apply uses under capture; the staged engine only when its row-block table for B already exists
     const int key = bh_tune_key(1, prec, B);
@@ -313,17 +339,15 @@ int bh_spmv_noalloc(bh_ctx* ctx, bh_ham* h, int prec, int B, const double* J, co
     if (var == 0 && h->rowblocks.find(B) == h->rowblocks.end()) var = 1;
     if (prec == BH_PREC_FP64) {
         SpmvArgs<double> a{h->D, h->row_ptr, h->words, h->diag, h->table, h->code_bits,
-                           sc, sc + SPMV_SCRATCH_LANES, static_cast<const double*>(x), static_cast<double*>(y), 1};
-        BH_TRY(spmv_launch(h, var, a, B, s));
+                           dJ, dU, static_cast<const double*>(x), static_cast<double*>(y), 1};
+        BH_TRY(spmv_launch(h, var, a, c, B, s));
     } else {
         SpmvArgs<float> a{h->D, h->row_ptr, h->words, h->diag, h->table, h->code_bits,
-                          sc, sc + SPMV_SCRATCH_LANES, static_cast<const float*>(x), static_cast<float*>(y), 1};
-        BH_TRY(spmv_launch(h, var, a, B, s));
+                          dJ, dU, static_cast<const float*>(x), static_cast<float*>(y), 1};
+        BH_TRY(spmv_launch(h, var, a, c, B, s));
     }
     BH_HIP(ctx, hipGetLastError());
-    // outside a capture the call returns with its work done (the host's J and U may be reused at once)
-    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    BH_HIP(ctx, hipStreamIsCapturing(s, &cs));
+    // outside a capture the call returns with its work done
     if (cs == hipStreamCaptureStatusNone) BH_HIP(ctx, hipStreamSynchronize(s));
     return BH_OK;
 }
@@ -336,25 +360,21 @@ int bh_spmv(bh_ctx* ctx, bh_ham* h, int prec, int B, const double* J, const doub
     BH_HIP(ctx, hipSetDevice(ctx->device));
     hipStream_t s = stream ? static_cast<hipStream_t>(stream) : ctx->stream;
     BH_TRY(bh_ham_prepare_locked(h, prec));
-    DevArray<double> dJ, dU;
-    BH_TRY(dJ.alloc(ctx, B));
-    BH_TRY(dU.alloc(ctx, B));
-    BH_HIP(ctx, hipMemcpyAsync(dJ.p, J, B * sizeof(double), hipMemcpyHostToDevice, s));
-    BH_HIP(ctx, hipMemcpyAsync(dU.p, U, B * sizeof(double), hipMemcpyHostToDevice, s));
+    const SpmvCoef c = bh_spmv_coef(J, U, B);
     {
         KTimer kt(ctx, "spmv", s);
         if (prec == BH_PREC_FP64) {
             SpmvArgs<double> a{h->D, h->row_ptr, h->words, h->diag, h->table, h->code_bits,
-                               dJ.p, dU.p, static_cast<const double*>(x), static_cast<double*>(y), 1};
-            BH_TRY(bh_apply(ctx, h, a, prec, B, s));
+                               nullptr, nullptr, static_cast<const double*>(x), static_cast<double*>(y), 1};
+            BH_TRY(bh_apply(ctx, h, a, c, prec, B, s));
         } else {
             SpmvArgs<float> a{h->D, h->row_ptr, h->words, h->diag, h->table, h->code_bits,
-                              dJ.p, dU.p, static_cast<const float*>(x), static_cast<float*>(y), 1};
-            BH_TRY(bh_apply(ctx, h, a, prec, B, s));
+                              nullptr, nullptr, static_cast<const float*>(x), static_cast<float*>(y), 1};
+            BH_TRY(bh_apply(ctx, h, a, c, prec, B, s));
         }
     }
     BH_HIP(ctx, hipGetLastError());
-    BH_HIP(ctx, hipStreamSynchronize(s));  // dJ/dU are freed on return
+    BH_HIP(ctx, hipStreamSynchronize(s));  // the call returns with its work done
     return BH_OK;
 }
 
@@ -399,24 +419,20 @@ int bh_spmv_bench(bh_ctx* ctx, bh_ham* h, int prec, int B, int reps, double* avg
     const size_t n = static_cast<size_t>(h->D) * B;
     const size_t es = prec == BH_PREC_FP64 ? 8 : 4;
     DevArray<uint8_t> dx, dy;
-    DevArray<double> dJ, dU;
     BH_TRY(dx.alloc(ctx, n * es));
     BH_TRY(dy.alloc(ctx, n * es));
-    BH_TRY(dJ.alloc(ctx, B));
-    BH_TRY(dU.alloc(ctx, B));
     std::vector<double> ones(B, 1.0);
-    BH_HIP(ctx, hipMemcpyAsync(dJ.p, ones.data(), B * 8, hipMemcpyHostToDevice, s));
-    BH_HIP(ctx, hipMemcpyAsync(dU.p, ones.data(), B * 8, hipMemcpyHostToDevice, s));
+    const SpmvCoef c = bh_spmv_coef(ones.data(), ones.data(), B);
     BH_HIP(ctx, hipMemsetAsync(dx.p, 0, n * es, s));
     auto launch = [&]() -> int {
         if (prec == BH_PREC_FP64) {
             SpmvArgs<double> a{h->D, h->row_ptr, h->words, h->diag, h->table, h->code_bits,
-                               dJ.p, dU.p, reinterpret_cast<const double*>(dx.p), reinterpret_cast<double*>(dy.p), 1};
-            return bh_apply(ctx, h, a, prec, B, s);
+                               nullptr, nullptr, reinterpret_cast<const double*>(dx.p), reinterpret_cast<double*>(dy.p), 1};
+            return bh_apply(ctx, h, a, c, prec, B, s);
         }
         SpmvArgs<float> a{h->D, h->row_ptr, h->words, h->diag, h->table, h->code_bits,
-                          dJ.p, dU.p, reinterpret_cast<const float*>(dx.p), reinterpret_cast<float*>(dy.p), 1};
-        return bh_apply(ctx, h, a, prec, B, s);
+                          nullptr, nullptr, reinterpret_cast<const float*>(dx.p), reinterpret_cast<float*>(dy.p), 1};
+        return bh_apply(ctx, h, a, c, prec, B, s);
     };
     BH_TRY(launch());  // warm-up (also builds the row blocks)
     hipEvent_t e0, e1;
