@@ -59,3 +59,25 @@ def test_spdm_ground_state_full_size(ctx):
     assert 1.0 / m < cf < 1.0 and 0.0 < K < 1.0
     h.close()
     b.close()
+
+
+@pytest.mark.parametrize("order", [bhx.ORDER_REFERENCE, bhx.ORDER_LEX])
+@pytest.mark.parametrize("m,n", [(1, 3), (2, 1), (4, 0), (5, 7), (12, 4), (16, 3), (17, 3), (3, 20), (18, 2), (3, 50), (2, 80)])
+def test_spdm_layouts(m, n, order):
+    """every packed-state layout, the last group of rows shorter than a group, amplitudes from the table and beyond it
+    (n > 62), one state to several workgroups; sums of at most D n terms: D eps of the largest entry, n"""
+    print(f"spdm m={m} n={n} order={order}", flush=True)
+    st, _, lex = O.basis(m, n)
+    with bhx.Context(0) as c:
+        b = c.basis(m, n, order)
+        phi = np.random.default_rng(m * n).standard_normal(b.D)
+        phi /= np.linalg.norm(phi)
+        want = O.spdm(st, phi)
+        mine = phi
+        if order == bhx.ORDER_LEX:  # position = lexicographic rank
+            mine = np.empty_like(phi)
+            mine[lex] = phi
+        got = b.spdm(mine)
+        b.close()
+    assert np.array_equal(got, got.T)
+    assert np.abs(got - want).max() <= max(b.D, 8) * 2.3e-16 * max(n, 1)
