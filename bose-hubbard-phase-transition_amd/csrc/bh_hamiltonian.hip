@@ -254,7 +254,8 @@ __global__ void __launch_bounds__(256) k_ham_stats(const int4* __restrict__ stat
 // i = NI blockIdx.y .. + NI - 1: a thread unranks its state once for all of them, gets the rank of b_i^+ b_j s as its own
 // plus a difference of two prefix sums (as k_ham_fill does), and keeps the sums of its NI m pairs in registers over all its
 // states; the wave is summed once at the end.  m = 12, n = 12: 2,290 us, when every pair of every state ranked its target site by
-// site and was summed over the wave, to 387 us (two waves per SIMD: the sums take 128 registers).
+// site and was summed over the wave, to 362 us (387 with four rows: the sums
+// then take 128 registers and two waves fit a SIMD).
 template <int NW, int BITS, int NI>
 __global__ void __launch_bounds__(256) k_spdm(int64_t D, int m, int n, const uint32_t* __restrict__ gg, int gsize,
                                               const double* __restrict__ phi, int nsq, double* __restrict__ part) {
@@ -755,7 +756,7 @@ int bh_spdm(bh_ctx* ctx, const bh_basis* b, const double* phi, double* rho) {
     }
 #define LAUNCH_SPDM(NW_, BITS_)                                                                                       \
     do {                                                                                                              \
-        constexpr int NI = PState<NW_, BITS_>::MAXM == 16 ? 4 : 2;                                                    \
+        constexpr int NI = PState<NW_, BITS_>::MAXM == 16 ? 2 : 1;                                                    \
         hipLaunchKernelGGL((k_spdm<NW_, BITS_, NI>), dim3(nb, (m + NI - 1) / NI), dim3(256), lds_bytes, s, D, m, n,   \
                            b->rank_tab, gsize, dphi, nsq, part);                                                      \
     } while (0)

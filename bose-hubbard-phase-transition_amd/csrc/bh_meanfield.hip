@@ -11,7 +11,7 @@
 // Arithmetic: every expression keeps one fixed operand order and the file's functions are compiled without
 // floating-point contraction, so each result is a fixed sequence of correctly rounded IEEE operations
 // (+, -, *, / and the sqrt(i) table computed on the host).  A ground state needs only a few O(2p+1) pivot
-// recurrences (no eigenvector, no per-thread arrays), so every point's state lives in registers.
+// recurrences (no eigenvector): a point's state lives in registers and one column of LDS (its diagonal).
 #include <algorithm>
 #include <cmath>
 #include <vector>
@@ -24,6 +24,7 @@ constexpr int MF_PMAX = 32;             // largest p a point may reach: h_MF on 
 constexpr int MF_NMAX = 2 * MF_PMAX + 1;
 constexpr int MF_WG = 256;
 constexpr int MF_GRID = 2048;           // workgroups of one launch: 8 per CU; later points are claimed
+constexpr int MF_NL = 16;               // diagonal entries a lane keeps in LDS (32 KB a workgroup); p <= 7, all but rare points
 
 __device__ __forceinline__ double mf_diag(int i, double mu, double w) {
 #pragma clang fp contract(off)
@@ -49,6 +50,42 @@ __device__ bool mf_pivots(int N, double mu, double w, double c2, double x, doubl
     }
     S = s;
     return true;
+}
+
+// 1 / u, correctly rounded, for a positive u with an exponent in [-511, 512]: the steps the compiler's IEEE division takes
+// for a numerator of 1 -- reciprocal estimate, two Newton steps, residual correction -- without its scaling and
+// fix-up, which change nothing there.
+__device__ __forceinline__ double mf_rcp(double u) {
+#pragma clang fp contract(off)
+    double y = __builtin_amdgcn_rcp(u);
+    y = fma(y, fma(-u, y, 1.0), y);
+    y = fma(y, fma(-u, y, 1.0), y);
+    return fma(fma(-u, y, 1.0), y, y);
+}
+
+// Range of a pivot, by its high word less 2^29: below MF_MID, positive with an exponent in [-511, 512]; from MF_NEG
+// below MF_TINY, negative; otherwise zero, tiny, huge or NaN.  The largest over a sweep tells what it met.
+constexpr unsigned MF_MID = 0x40000000u, MF_NEG = 0x60000000u, MF_TINY = 0xe0000000u;
+__device__ __forceinline__ unsigned mf_range(double u) { return static_cast<unsigned>(__double2hiint(u)) - 0x20000000u; }
+
+// mf_pivots on the entries d[0], d[MF_WG], ... of this lane in LDS, the same operations without a branch per pivot:
+// 1 all pivots positive, 0 one is not (S then unused), -1 left to mf_pivots.  A sweep is one chain of dependent
+// FP64 operations, alone on its SIMD for most of the launch, so its length in instructions is the kernel's time.
+__device__ __forceinline__ int mf_sweep(int N, const double* d, double c2, double x, double& S) {
+#pragma clang fp contract(off)
+    double u = d[0] - x, du = -1.0, r = mf_rcp(u), s = du * r, f = 0.0;
+    unsigned t = mf_range(u);
+    for (int i = 1; i < N; ++i) {
+        f = f + 1.0;
+        const double ee = c2 * f;
+        du = -1.0 + ee * du * r * r;
+        u = (d[i * MF_WG] - x) - ee * r;
+        t = max(t, mf_range(u));
+        r = mf_rcp(u);
+        s = s + du * r;
+    }
+    S = s;
+    return t < MF_MID ? 1 : (t >= MF_NEG && t < MF_TINY ? 0 : -1);
 }
 
 // Logarithmic derivatives of det(T - x I) in x and in the coupling scale c (diagonal held fixed) at two points
@@ -89,7 +126,7 @@ __device__ void mf_logdet_deriv2(int N, double mu, double w, double c2, double t
 }
 
 // Ground state of h_MF(psi, p):  d_i = -mu i + i(i-1)/2 + q J psi^2,  h(i, i+1) = c sqrt(i+1), c = -q J psi.
-// Returns its energy and sf = <phi|a|phi>, all in registers (no eigenvector is formed).
+// Returns its energy, in registers and the lane's LDS column d (no eigenvector is formed).
 // Energy: Newton's iteration on ln det(T - x I) from below (x <- x - 1/S).  Every root is real, so each exact
 // step from below the lowest root stays below it and the iterates rise monotonically to it (quadratically
 // once close).  Starts at `hint` when its pivots are all positive (the previous p's eigenvalue less 1e-3
@@ -97,48 +134,59 @@ __device__ void mf_logdet_deriv2(int N, double mu, double w, double c2, double t
 // rejected hint, lies at or above the root.  An iterate without all pivots positive, or a step reaching hi,
 // can only come from rounding at the root: that iterate (resp. hi) is returned, as is the last iterate when
 // a step no longer moves x.
-// <a>: Hellmann-Feynman, d lambda/dc = 2 sum_i sqrt(i+1) phi_i phi_{i+1} = 2 <a> and d lambda/dc =
-// -(d ln det/dc) / (d ln det/dx) as x -> lambda; the ratio is taken at lambda - delta and lambda - 2 delta,
-// delta = 1e-9 (|lambda| + 1), and extrapolated linearly to lambda (O(delta^2) error).
-// c = 0 (diagonal h): the first smallest diagonal entry and <a> = 0.
-__device__ double mf_ground(double psi, int p, double mu, double J, int q, const double* __restrict__ sq, double hint,
-                            double& sf) {
+// c = 0 (diagonal h): the first smallest diagonal entry.
+__device__ double mf_ground(double psi, int p, double mu, double J, int q, const double* __restrict__ sq, double hint, double* d) {
 #pragma clang fp contract(off)
     const int N = 2 * p + 1;
     const double c = static_cast<double>(-q) * J * psi;
     const double w = static_cast<double>(q) * J * psi * psi;
-    double lo = 0.0, hi = 0.0;
+    double lo = 0.0, hi = 0.0, top = 0.0;
     for (int i = 0; i < N; ++i) {
-        const double d = mf_diag(i, mu, w);
+        const double di = mf_diag(i, mu, w);
+        if (i < MF_NL) d[i * MF_WG] = di;
         const double a0 = i > 0 ? fabs(c * sq[i]) : 0.0;
         const double a1 = i < N - 1 ? fabs(c * sq[i + 1]) : 0.0;
-        const double g = d - a0 - a1;
+        const double g = di - a0 - a1;
         if (i == 0 || g < lo) lo = g;
-        if (i == 0 || d < hi) hi = d;
+        if (i == 0 || di < hi) hi = di;
+        top = fmax(top, fabs(di));
     }
-    sf = 0.0;
     if (c == 0.0) return hi;
-    const double c2 = c * c, tc = 2.0 * c;
+    const double c2 = c * c;
+    // the sweep without range checks on d_i - x: no pivot above 2^512 while those before it are positive
+    const bool fast = N <= MF_NL && top < 0x1p400 && fabs(lo) < 0x1p400;
+    auto pivots = [&](double x, double& S) -> bool {
+        if (fast) {
+            const int k = mf_sweep(N, d, c2, x, S);
+            if (k >= 0) return k == 1;
+        }
+        return mf_pivots(N, mu, w, c2, x, S);
+    };
     double S = 0.0;
     // the start: the hint when its pivots are all positive, else the Gershgorin bound (moved down if rounding
-    // put it at the eigenvalue)
+    // put it at the eigenvalue).  Each evaluation is one step of Newton's iteration, so its S is kept.
     double xk = lo;
-    bool have_start = false;
+    bool have = false;
     if (hint > lo && hint < hi) {
-        if (mf_pivots(N, mu, w, c2, hint, S)) {
+        if (pivots(hint, S)) {
             xk = hint;
-            have_start = true;
+            have = true;
         } else {
             hi = hint;
         }
     }
-    if (!have_start) {
-        for (int t = 0; t < 64 && !mf_pivots(N, mu, w, c2, lo, S); ++t) lo = lo - (fabs(lo) + 1.0);
+    if (!have) {
+        for (int t = 0; t < 64; ++t) {
+            have = pivots(lo, S);
+            if (have) break;
+            lo = lo - (fabs(lo) + 1.0);
+        }
         xk = lo;
     }
     double lam = xk;
     for (int it = 0; it < 200; ++it) {
-        if (!mf_pivots(N, mu, w, c2, xk, S)) break;  // a Newton iterate at the root within rounding
+        if (!have && !pivots(xk, S)) break;  // a Newton iterate at the root within rounding
+        have = false;
         const double xn = xk - 1.0 / S;
         if (!(xn < hi)) {  // the root lies at hi within rounding
             lam = hi;
@@ -148,6 +196,20 @@ __device__ double mf_ground(double psi, int p, double mu, double J, int q, const
         xk = xn;
         lam = xk;
     }
+    return lam;
+}
+
+// <a> of the ground state with energy lam: Hellmann-Feynman, d lambda/dc = 2 sum_i sqrt(i+1) phi_i phi_{i+1} = 2 <a> and
+// d lambda/dc = -(d ln det/dc) / (d ln det/dx) as x -> lambda; the ratio is taken at lambda - delta and
+// lambda - 2 delta, delta = 1e-9 (|lambda| + 1), and extrapolated linearly to lambda (O(delta^2) error).
+// Only the last p of an iteration needs it.  c = 0 (diagonal h): 0.
+__device__ double mf_order(double psi, int p, double mu, double J, int q, double lam) {
+#pragma clang fp contract(off)
+    const int N = 2 * p + 1;
+    const double c = static_cast<double>(-q) * J * psi;
+    const double w = static_cast<double>(q) * J * psi * psi;
+    if (c == 0.0) return 0.0;
+    const double c2 = c * c, tc = 2.0 * c;
     double delta = 1e-9 * (fabs(lam) + 1.0);
     for (int t = 0; t < 8; ++t) {
         double sx1, sc1, sx2, sc2;
@@ -156,12 +218,11 @@ __device__ double mf_ground(double psi, int p, double mu, double J, int q, const
         if (ok1 && ok2) {
             const double f1 = -0.5 * sc1 / sx1;
             const double f2 = -0.5 * sc2 / sx2;
-            sf = 2.0 * f1 - f2;
-            break;
+            return 2.0 * f1 - f2;
         }
         delta = 2.0 * delta;
     }
-    return lam;
+    return 0.0;
 }
 
 // the start for p + 1 after the eigenvalue e of p
@@ -178,6 +239,10 @@ __device__ __forceinline__ double mf_hint(double e) {
 // neighbours; per-lane refill keeps the other lanes of the wavefront busy meanwhile.  Each lane starts at
 // its global thread index; later points are claimed in wavefront batches from *next (zero at launch), offset
 // by the number of threads.  A wavefront leaves the loop when none of its lanes holds a point.
+// The launch ends with the slowest point's chain: its 2,178 iterations take 35 ms alone (59 before a sweep lost its
+// branches and an iteration its order parameters of all p but the last and one sweep of each), the reference's
+// 1000 x 1000 grid 68 ms (92).  Handing the points left after 64, 256 and 768 iterations to launches with one
+// wavefront per SIMD and few lanes each was slower (75 ms).
 __global__ void __launch_bounds__(MF_WG) k_scmf(int64_t npts, const double* __restrict__ mu_in,
                                                 const double* __restrict__ J_in, const double* __restrict__ psi0,
                                                 int q, double eps, int max_outer, int pmax,
@@ -186,12 +251,14 @@ __global__ void __launch_bounds__(MF_WG) k_scmf(int64_t npts, const double* __re
                                                 int32_t* __restrict__ p_out, unsigned long long* __restrict__ next) {
 #pragma clang fp contract(off)
     __shared__ double sq[MF_NMAX + 1];
+    __shared__ double dl[MF_NL * MF_WG];
     for (int i = threadIdx.x; i <= MF_NMAX; i += MF_WG) sq[i] = sq_in[i];
     __syncthreads();
+    double* d = dl + threadIdx.x;
     const int64_t nthreads = static_cast<int64_t>(gridDim.x) * MF_WG;
     const int lane = static_cast<int>(__lane_id());
     int64_t k = static_cast<int64_t>(blockIdx.x) * MF_WG + threadIdx.x;
-    double mu = 0.0, J = 0.0, psi = 0.0, e0 = 0.0, sf = 0.0;
+    double mu = 0.0, J = 0.0, psi = 0.0, e0 = 0.0;
     int p = 1, outer = 1;
     bool have = k < npts, exhausted = !have;
     if (have) {
@@ -201,7 +268,7 @@ __global__ void __launch_bounds__(MF_WG) k_scmf(int64_t npts, const double* __re
     }
     for (;;) {
         if (have) {
-            const double e = mf_ground(psi, p, mu, J, q, sq, p == 1 ? -INFINITY : mf_hint(e0), sf);
+            const double e = mf_ground(psi, p, mu, J, q, sq, p == 1 ? -INFINITY : mf_hint(e0), d);
             int status = -1;
             if (p == 1) {
                 e0 = e;
@@ -215,6 +282,7 @@ __global__ void __launch_bounds__(MF_WG) k_scmf(int64_t npts, const double* __re
                     else
                         ++p;
                 } else {
+                    const double sf = mf_order(psi, p, mu, J, q, e);
                     const double dpsi = fabs(sf - psi);
                     psi = sf;
                     if (dpsi <= eps) {

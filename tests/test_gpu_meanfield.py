@@ -123,3 +123,16 @@ def test_scmf_full_size_phase_diagram(ctx):
     idx = np.random.default_rng(9).choice(mu.size, 1500, replace=False)
     st, psi, it, p = oracle_all(mu[idx], J[idx], psi0[idx], eps)
     assert np.array_equal(r["psi"][idx], psi) and np.array_equal(r["iters"][idx], it)
+
+
+@pytest.mark.parametrize("mu,J,q", [(6.5, 0.3, 2), (9.2, 0.4, 2), (0.5, 1e-200, 1), (1e120, 0.1, 1), (1e160, 0.1, 1), (-1e155, 3.0, 1), (3.0, 1e3, 4)])
+def test_scmf_wide_and_extreme_points_bitwise(ctx, mu, J, q):
+    """points that need more occupations than a lane keeps on chip (p > 7), and pivots outside the range of the branch-free
+    sweep: the same bits as the oracle's scalar restatement"""
+    print(f"scmf mu={mu} J={J} q={q}", flush=True)
+    psi0 = np.array([0.3, 1e-3, 2.5, 0.0])
+    r = ctx.mean_field(np.full(4, mu), np.full(4, J), psi0, q=q, eps=1e-7, max_outer=50)
+    for i in range(4):
+        st, psi, it, pl = O.scmf(mu, J, q, psi0[i], 1e-7, max_outer=50)
+        assert (r["status"][i], r["iters"][i], r["p"][i]) == (st, it, pl), i
+        assert np.array_equal(r["psi"][i:i + 1], np.array([psi]), equal_nan=True), (r["psi"][i], psi)
