@@ -914,17 +914,19 @@ __global__ void __launch_bounds__(LZ_RED_WG) k_lz_beta(LzState st, const double*
 }
 
 // R1 over many K1 workgroups: one workgroup per value (blockIdx.x = v), each thread summing a strided
-// subset of the partials in a fixed order, then a fixed tree over the workgroup.  Only the alpha sums
+// subset of the partials in a fixed order (nwg rows of the first nmin values, nwg_so of the others), then a fixed
+// tree over the workgroup.  Only the alpha sums
 // (v < nmin) unless the step is exact (then also the locked-vector sums).
 template <int B>
-__global__ void __launch_bounds__(LZ_RED_WG) k_lz_reduce_wide(LzState st, const double* __restrict__ part, int nwg,
+__global__ void __launch_bounds__(LZ_RED_WG) k_lz_reduce_wide(LzState st, const double* __restrict__ part, int nwg, int nwg_so,
                                                               int nv, int nmin, int so_any, double* __restrict__ out) {
     __shared__ double red[LZ_RED_WG / 64];
     const int v = blockIdx.x;
     const int nvv = (so_any ? st.so[0] != 0 : st.so[0] == 1) ? nv : nmin;
     if (v >= nvv) return;  // uniform over the workgroup
     double s = 0.0;
-    for (int w = threadIdx.x; w < nwg; w += LZ_RED_WG) s += part[static_cast<size_t>(w) * nv + v];
+    const int rows = v < nmin ? nwg : nwg_so;
+    for (int w = threadIdx.x; w < rows; w += LZ_RED_WG) s += part[static_cast<size_t>(w) * nv + v];
 #pragma unroll
     for (int o = 32; o >= 1; o >>= 1) s += __shfl_xor(s, o, 64);
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
@@ -1136,7 +1138,8 @@ __global__ void __launch_bounds__(LZ_WG) k_lz_dots(const YT* __restrict__ Y, con
 // value q < nv: <Y_i, Y_q> and value nv + q: <Y_i, HY_q> (reduced by k_lz_reduce mode 0)
 // Rows i0 .. i0 + NI - 1 of the Gram matrices of the finish, per lane: G(i, q) = <y_i, y_q> and
 // A(i, q) = <y_i, H y_q> for q < nv <= NV, as per-workgroup partials of the values ((i - i0) 2 + w) NV + q
-// (w = 0: G, 1: A); each thread reads its NI row elements once and every column element once.
+// (w = 0: G, 1: A); each thread reads its NI row elements once and every column element from q = i0 on once (both
+// matrices are symmetric: the host takes the entries below the diagonal from above it).
 template <int B, int NV, int NI>
 __global__ void __launch_bounds__(LZ_WG) k_lz_gram_rows(const double* __restrict__ Y, const double* __restrict__ HY, int64_t D,
                                                         int nv, int i0, double* part) {
@@ -1159,7 +1162,7 @@ __global__ void __launch_bounds__(LZ_WG) k_lz_gram_rows(const double* __restrict
         for (int ii = 0; ii < NI; ++ii) yi[ii] = i0 + ii < nv ? Y[static_cast<int64_t>(i0 + ii) * vs + idx] : 0.0;
 #pragma unroll
         for (int q = 0; q < NV; ++q)
-            if (q < nv) {
+            if (q < nv && q >= i0) {
                 const double yq = Y[static_cast<int64_t>(q) * vs + idx], hq = HY[static_cast<int64_t>(q) * vs + idx];
 #pragma unroll
                 for (int ii = 0; ii < NI; ++ii) {
@@ -1413,12 +1416,12 @@ int lz_refine_steps() {
     return d;
 }
 
-// Steps enqueued at an analysis before the host analyses (the device runs them meanwhile): one captured
-// graph's worth by default, BHX_SPEC=0 turns the overlap off.
-int lz_spec_steps() {
-    static int d = [] {
+// Steps enqueued at an analysis before the host analyses (the device runs them meanwhile); BHX_SPEC=0 turns the overlap
+// off.
+bool lz_spec_on() {
+    static bool d = [] {
         const char* e = std::getenv("BHX_SPEC");
-        return (e && std::strcmp(e, "0") == 0) ? 0 : LZ_GRAPH_STEPS;
+        return !(e && std::strcmp(e, "0") == 0);
     }();
     return d;
 }
@@ -1854,7 +1857,7 @@ class LzEngine final : public LzEngineBase {
         // basis vectors untouched; a lane whose basis is full runs no speculative step.
         jsync = jl;
         totsync = tot;
-        if (speculate()) BH_TRY(run(lz_spec_steps()));
+        if (speculate()) BH_TRY(run(spec_steps()));
         struct HostClock {  // adds the host time of this analysis to the engine's profile on return
             LzEngine* e;
             std::chrono::steady_clock::time_point t;
@@ -2266,7 +2269,11 @@ class LzEngine final : public LzEngineBase {
                 }
                 BH_TRY(rc0);
             }
-            BH_TRY(form_vectors(njb, nvf, C, Yfp, vs));
+            // slots below every lane's frozen count hold frozen vectors only (copied below)
+            int nfmin = nvf;
+            for (int b : lanes) nfmin = std::min(nfmin, nf[b]);
+            if (static_cast<int>(lanes.size()) < B) nfmin = 0;
+            BH_TRY(form_vectors(njb, nvf, C, Yfp, vs, nfmin));
             if (nfmax > 0) {
                 BH_HIP(ctx, hipMemcpyAsync(dnj.p, nf.data(), B * sizeof(int), hipMemcpyHostToDevice, s));
                 hipLaunchKernelGGL((k_lz_copy_frozen<XT, B>), dim3(static_cast<unsigned>((vs + 255) / 256)), dim3(256), 0, s, Y,
@@ -2654,8 +2661,14 @@ class LzEngine final : public LzEngineBase {
         for (int b : lanes) {
             const int n = std::min(nt[b], nvf);
             if (n == 0) continue;
-            auto G = [&](int i, int q) { return g[(static_cast<size_t>(i) * 2 * nvf + q) * B + b]; };
-            auto A = [&](int i, int q) { return g[(static_cast<size_t>(i) * 2 * nvf + nvf + q) * B + b]; };
+            // up to LZ_NVMAX candidates the entries on and above the diagonal are there
+            const bool half = nvf <= LZ_NVMAX;
+            auto at = [&](int i, int q, int w) {
+                if (half && q < i) std::swap(i, q);
+                return g[(static_cast<size_t>(i) * 2 * nvf + static_cast<size_t>(w) * nvf + q) * B + b];
+            };
+            auto G = [&](int i, int q) { return at(i, q, 0); };
+            auto A = [&](int i, int q) { return at(i, q, 1); };
             std::vector<double> Gm(n * n), gw(n), Ug(n * n);
             for (int i = 0; i < n; ++i)
                 for (int q = 0; q < n; ++q) Gm[i * n + q] = 0.5 * (G(i, q) + G(q, i));
@@ -2721,7 +2734,10 @@ class LzEngine final : public LzEngineBase {
     // Speculative steps keep the device busy during a host analysis at every size: an analysis takes 0.1 to 0.4 ms a
     // lane, eight steps of a small sector 0.2 to 0.7 ms.  A lane that its analysis changes wastes them (three passes
     // of a D = 6,435 solve: 24 of 345 steps).
-    bool speculate() const { return lz_spec_steps() > 0; }
+    bool speculate() const { return lz_spec_on(); }
+    // A lane that locks, restarts or ends at the analysis loses the steps it has run past it, so there are only as many as
+    // an analysis takes: eight up to 4M elements, fewer beyond, by size alone (sums do not depend on the timing).
+    int spec_steps() const { return static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(LZ_GRAPH_STEPS, (int64_t(32) << 20) / vs))); }
     // orthogonalisation variant of the next steps: the smallest of 0, 4, 8, 16 locked vectors that covers every
     // iterating lane's current set (a lane's set shrinks back to its frozen vectors at a deflation); none under
     // full reorthogonalisation, whose steps project out the frozen vectors themselves
@@ -2740,7 +2756,10 @@ class LzEngine final : public LzEngineBase {
     void set_k1(int var) {
         k1v = var;
         grid_k1 = var == 0 ? grid_rb : static_cast<int>((D + k1_rows(var) - 1) / k1_rows(var));
-        rpw_so = (D + grid_k1 - 1) / grid_k1;
+        // the exact steps' dot products: rows of K1's partial sums, but no more workgroups than fill the chip, since
+        // most steps only find that there is nothing to do (6 us for 10,564 of them)
+        grid_so = std::min(grid_k1, LZ_K2_GRID);
+        rpw_so = (D + grid_so - 1) / grid_so;
     }
     // LDS of a row-lane variant: the table, and on the row-tile engine (V = B) each wave's words
     size_t k1_shm(int V) const { return shm + (V == B ? static_cast<size_t>(LZ_WG / 64) * tile_cap * sizeof(uint32_t) : 0); }
@@ -2787,9 +2806,9 @@ class LzEngine final : public LzEngineBase {
         }
         if (LM > 0) {
             KTimer kt(ctx, "lanczos_sodots", s);
-            if (LM == 4) hipLaunchKernelGGL((k_lz_sodots<XT, B, 4>), dim3(grid_k1), dim3(LZ_WG), 0, s, a, rpw_so, nv);
-            else if (LM == 8) hipLaunchKernelGGL((k_lz_sodots<XT, B, 8>), dim3(grid_k1), dim3(LZ_WG), 0, s, a, rpw_so, nv);
-            else hipLaunchKernelGGL((k_lz_sodots<XT, B, 16>), dim3(grid_k1), dim3(LZ_WG), 0, s, a, rpw_so, nv);
+            if (LM == 4) hipLaunchKernelGGL((k_lz_sodots<XT, B, 4>), dim3(grid_so), dim3(LZ_WG), 0, s, a, rpw_so, nv);
+            else if (LM == 8) hipLaunchKernelGGL((k_lz_sodots<XT, B, 8>), dim3(grid_so), dim3(LZ_WG), 0, s, a, rpw_so, nv);
+            else hipLaunchKernelGGL((k_lz_sodots<XT, B, 16>), dim3(grid_so), dim3(LZ_WG), 0, s, a, rpw_so, nv);
         }
     }
     // Autotuner of K1, run once per (sector, precision, batch width) on the engine's first steps (the
@@ -2868,7 +2887,7 @@ class LzEngine final : public LzEngineBase {
             KTimer kt(ctx, "lanczos_reorth", s);
             const bool direct = grid_k1 * B <= 4096;
             if (!direct)
-                hipLaunchKernelGGL((k_lz_reduce_wide<B>), dim3(B), dim3(LZ_RED_WG), 0, s, st, part.p, grid_k1, B, B, 0, st.sums);
+                hipLaunchKernelGGL((k_lz_reduce_wide<B>), dim3(B), dim3(LZ_RED_WG), 0, s, st, part.p, grid_k1, grid_k1, B, B, 0, st.sums);
             const int nt = frs.rows / LZ_FR_T;
             const int gd = frs.nR * std::min(nt, std::max(1, LZ_FR_GRID / frs.nR));
             hipLaunchKernelGGL((k_lz_fr_dots<B>), dim3(gd), dim3(LZ_FR_WG), 0, s, a, frs, direct ? grid_k1 : 0, dd.p);
@@ -2898,7 +2917,7 @@ class LzEngine final : public LzEngineBase {
         {
             KTimer kt(ctx, "lanczos_reduce", s);
             const int nv = (1 + 2 * LM) * B;
-            hipLaunchKernelGGL((k_lz_reduce_wide<B>), dim3(nv), dim3(LZ_RED_WG), 0, s, st, part.p, grid_k1, nv, B, 0, st.sums);
+            hipLaunchKernelGGL((k_lz_reduce_wide<B>), dim3(nv), dim3(LZ_RED_WG), 0, s, st, part.p, grid_k1, grid_so, nv, B, 0, st.sums);
         }
         {
             KTimer kt(ctx, "lanczos_update", s);
@@ -2910,7 +2929,7 @@ class LzEngine final : public LzEngineBase {
         {
             KTimer kt(ctx, "lanczos_reduce", s);
             const int nv2 = (1 + LM) * B;
-            hipLaunchKernelGGL((k_lz_reduce_wide<B>), dim3(nv2), dim3(LZ_RED_WG), 0, s, st, part.p, grid_k2, nv2, B, 1,
+            hipLaunchKernelGGL((k_lz_reduce_wide<B>), dim3(nv2), dim3(LZ_RED_WG), 0, s, st, part.p, grid_k2, grid_k2, nv2, B, 1,
                                sums2.p);
             hipLaunchKernelGGL((k_lz_beta<B>), dim3(1), dim3(LZ_RED_WG), 0, s, st, sums2.p, nv2, cap, eps_store,
                                lz_so_always());
@@ -2932,9 +2951,9 @@ class LzEngine final : public LzEngineBase {
         *out = own.p;
         return BH_OK;
     }
-    // C holds rows t < max(njb) of [(t * nv + i) * B + b]
+    // C holds rows t < max(njb) of [(t * nv + i) * B + b]; outputs first .. nv - 1 are formed
     template <typename OT>
-    int form_vectors(const std::vector<int>& njb, int nv, const std::vector<double>& C, OT* out, int64_t os) {
+    int form_vectors(const std::vector<int>& njb, int nv, const std::vector<double>& C, OT* out, int64_t os, int first = 0) {
         int njmax = 0;
         for (int b = 0; b < B; ++b) njmax = std::max(njmax, njb[b]);
         if (C.size() < static_cast<size_t>(njmax) * nv * B) return bh_set_error(ctx, BH_EINVAL, "ritz: coefficient rows");
@@ -2945,7 +2964,7 @@ class LzEngine final : public LzEngineBase {
         {
             KTimer kt(ctx, "lanczos_ritz", s);
             const int64_t per_wg = 256 * LZ_RZ_R;
-            for (int i0 = 0; i0 < nv; i0 += LZ_RZ_G)
+            for (int i0 = first; i0 < nv; i0 += LZ_RZ_G)
                 hipLaunchKernelGGL((k_lz_ritz<XT, OT, B>), dim3(static_cast<unsigned>((vs + per_wg - 1) / per_wg)), dim3(256), 0,
                                    s, V, vs, dnj.p, njmax, dC.p, nv, i0, std::min(LZ_RZ_G, nv - i0), out, os);
         }
@@ -3321,7 +3340,7 @@ class LzEngine final : public LzEngineBase {
     LzFrSplit frs;
     LzState st{};
     LzArgs<XT> a{};
-    int k1v = 1, grid_rb = 1, grid_rl = 1, grid_k1 = 1, grid_k2 = 1;
+    int k1v = 1, grid_rb = 1, grid_rl = 1, grid_k1 = 1, grid_k2 = 1, grid_so = 1;
     bool staged_ok = false, tuned = false;
     int64_t rpw_so = 1, nrblk = 0;
     const int32_t* rblk = nullptr;
