@@ -136,3 +136,22 @@ def test_scmf_wide_and_extreme_points_bitwise(ctx, mu, J, q):
         st, psi, it, pl = O.scmf(mu, J, q, psi0[i], 1e-7, max_outer=50)
         assert (r["status"][i], r["iters"][i], r["p"][i]) == (st, it, pl), i
         assert np.array_equal(r["psi"][i:i + 1], np.array([psi]), equal_nan=True), (r["psi"][i], psi)
+
+
+@pytest.mark.parametrize("npts", [1, 5, 255, 5121, 9001, 330001])
+def test_scmf_order_of_work_does_not_show(ctx, npts):
+    """one point to a wavefront, a few, and points dealt out by class and claimed: every point's result is that of the
+    oracle, and the same bits wherever it stands in the batch"""
+    print(f"scmf npts={npts}", flush=True)
+    rng = np.random.default_rng(npts)
+    mu, J, psi0 = rng.uniform(-0.5, 4, npts), rng.uniform(0, 0.25, npts), rng.uniform(0, 1, npts)
+    mu[::97], J[::89] = np.round(mu[::97]), 0.0
+    r = ctx.mean_field(mu, J, psi0, eps=1e-5)
+    perm = rng.permutation(npts)
+    w = ctx.mean_field(mu[perm], J[perm], psi0[perm], eps=1e-5)
+    for key in ("psi", "status", "iters", "p"):
+        assert np.array_equal(w[key], r[key][perm]), key
+    idx = rng.choice(npts, min(npts, 200), replace=False)
+    st, psi, it, p = oracle_all(mu[idx], J[idx], psi0[idx], 1e-5)
+    assert np.array_equal(r["psi"][idx], psi) and np.array_equal(r["iters"][idx], it)
+    assert np.array_equal(r["status"][idx], st) and np.array_equal(r["p"][idx], p)
