@@ -26,7 +26,7 @@
 namespace {
 
 using Clock = std::chrono::steady_clock;
-constexpr int64_t SRV_SMALL_D = 1 << 15;  // sectors driven to completion within a pass (see worker_loop)
+constexpr int64_t SRV_SMALL_D = 1 << 15;  // sectors driven together for several chunks a pass (see worker_loop)
 constexpr double SRV_SMALL_MS = 5.0;
 using SectorKey = std::tuple<int, int, int, int, int>;  // kind, Lx, Ly, periodic, n
 
@@ -385,11 +385,32 @@ void harvest(bh_server* S, Sector& sc, int p) {
     sc.last_use = S->now();
 }
 
+// One engine, unless its chunk is still on its stream: analysed (finished lanes retired), refilled from its queue and
+// given its next chunk.  Returns whether anything was done.
+bool advance(bh_server* S, Sector& sc, int p) {
+    bool did = false;
+    if (sc.inflight[p]) {
+        if (hipStreamQuery(sc.stream[p]) == hipErrorNotReady) return false;
+        sc.inflight[p] = false;
+        did = true;
+        harvest(S, sc, p);
+    }
+    admit_queued(S, sc, p);
+    if (!(sc.eng[p] && sc.eng[p]->active() > 0)) return did;
+    const int rc = sc.eng[p]->run(sc.eng[p]->suggest_chunk());
+    if (rc != BH_OK) fail_engine(S, sc, p, rc);
+    else sc.inflight[p] = true;
+    return true;
+}
+
 // The engines run independently: each pass of the loop visits every sector engine; one whose chunk is still
-// on its stream is skipped, one whose stream is idle is analysed (finished lanes retired), refilled from its
-// queue and given its next chunk at once.  A small sector thus cycles through its steps while a large one's
-// chunk is running, and no engine waits for another's.  Each engine still runs the same sequence of chunks
-// and analyses, so a request's result does not depend on the other requests.
+// on its stream is skipped, one whose stream is idle is analysed, refilled and given its next chunk at once.  A small
+// sector thus cycles through its steps while a large one's chunk is running, and no engine waits for another's.
+// A small sector's chunks take well under a millisecond, less than the host work of a pass over the large ones (CSR
+// builds, tuning, finishes), so a pass goes round the small sectors again and again, up to SRV_SMALL_MS for each of them;
+// their chunks run side by side on their streams (24 requests over eight sectors: 177 ms one sector after the other,
+// 147 so).  Each engine still runs the same sequence of chunks and analyses, so a request's result does not depend
+// on the other requests.
 void worker_loop(bh_server* S) {
     (void)hipSetDevice(S->ctx->device);
     for (;;) {
@@ -415,37 +436,32 @@ void worker_loop(bh_server* S) {
             }
         }
         bool progressed = false;
-        for (auto it = S->sectors.begin(); it != S->sectors.end(); ++it) {
-            Sector& sc = *it->second;
-            for (int p = 0; p < 2; ++p) {
-                // a small sector's chunks take well under a millisecond: it is driven chunk after chunk for up
-                // to SRV_SMALL_MS instead of one chunk per pass, so that it does not wait for the host work of
-                // every other sector (CSR builds, tuning, finishes) between its chunks
-                const bool small = sc.ham && sc.ham->D <= SRV_SMALL_D;
-                const auto t0 = Clock::now();
-                for (;;) {
-                    if (sc.inflight[p]) {
-                        if (small)
-                            (void)hipStreamSynchronize(sc.stream[p]);
-                        else if (hipStreamQuery(sc.stream[p]) == hipErrorNotReady)
-                            break;
-                        sc.inflight[p] = false;
-                        progressed = true;
-                        harvest(S, sc, p);
-                    }
-                    admit_queued(S, sc, p);
-                    if (!(sc.eng[p] && sc.eng[p]->active() > 0)) break;
-                    const int rc = sc.eng[p]->run(sc.eng[p]->suggest_chunk());
-                    if (rc != BH_OK) {
-                        fail_engine(S, sc, p, rc);
-                        progressed = true;
-                        break;
-                    }
-                    sc.inflight[p] = true;
-                    progressed = true;
-                    if (!small || std::chrono::duration<double, std::milli>(Clock::now() - t0).count() > SRV_SMALL_MS) break;
-                }
+        std::vector<Sector*> small;
+        for (auto& kv : S->sectors) {
+            Sector& sc = *kv.second;
+            if (sc.ham && sc.ham->D <= SRV_SMALL_D) {
+                small.push_back(&sc);
+                continue;
             }
+            for (int p = 0; p < 2; ++p) progressed |= advance(S, sc, p);
+        }
+        for (const auto t0 = Clock::now();;) {
+            bool did = false;
+            Sector* wait = nullptr;
+            int wp = 0, on = 0;
+            for (Sector* sc : small)
+                for (int p = 0; p < 2; ++p) {
+                    did |= advance(S, *sc, p);
+                    if (!sc->inflight[p]) continue;
+                    ++on;
+                    if (!wait) {
+                        wait = sc;
+                        wp = p;
+                    }
+                }
+            progressed |= did;
+            if (on == 0 || std::chrono::duration<double, std::milli>(Clock::now() - t0).count() > on * SRV_SMALL_MS) break;
+            if (!did) (void)hipStreamSynchronize(wait->stream[wp]);  // nothing to do until a chunk completes
         }
         S->hbm_used = S->ctx->used;
         if (!progressed) std::this_thread::sleep_for(std::chrono::microseconds(20));
