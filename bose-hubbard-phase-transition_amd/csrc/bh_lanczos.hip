@@ -57,6 +57,7 @@ constexpr int LZ_GRAPH_STEPS = 8;  // Lanczos steps per captured HIP graph
 constexpr int LZ_K2_GRID = 1024;   // K2 workgroups at most (rows of partial sums for R2; 512 and 2048 measured slower)
 constexpr int LZ_K1_TILES = 4;         // row groups per K1 workgroup on the row-lane engine at most
 constexpr int LZ_K1_FILL = 512;        // K1 workgroups below which it takes fewer row groups (two per CU)
+constexpr int LZ_DIRECT_B = 4;         // lanes up to which K2 may add up K1's partial sums itself
 constexpr int LZ_TUNE_REPS = 3;        // timed launches per K1 variant in the autotuner
 constexpr int LZ_CHECK_MIN = 4;        // fewest steps between two analyses of a lane
 constexpr int64_t LZ_PART_BYTES = 64ll << 20;  // partial sums of the staged K1 (more workgroups than grid_rl)
@@ -365,18 +366,45 @@ __global__ void __launch_bounds__(LZ_WG) k_lz_sodots(LzArgs<XT> a, int64_t rows_
 // step reads each locked vector once instead of twice (K1 skips them).
 // Eight locked vectors: held to 64 VGPRs (eight waves per SIMD, the 1024-workgroup grid in one round; 20 bytes
 // of spills per lane) -- 131 us per launch at the chain m=12 sector against 138 us at 66 VGPRs and seven waves.
-template <typename XT, int B, int LM>
-__global__ void __launch_bounds__(LZ_WG) __attribute__((amdgpu_waves_per_eu(LM == 8 ? 8 : 1))) k_lz_b(LzArgs<XT> a) {
+// DIRECT: K1's partial sums (nk1 rows of alpha, nso of the dot products of an exact step) are added up here, by every
+// workgroup in the same order, and recorded by workgroup 0; else R1 has done it.  part2: this kernel's partials,
+// apart from K1's where those are read here.
+template <typename XT, int B, int LM, bool DIRECT>
+__global__ void __launch_bounds__(LZ_WG) __attribute__((amdgpu_waves_per_eu(LM == 8 ? 8 : 1))) k_lz_b(LzArgs<XT> a, int nk1, int nso,
+                                                                                                      double* __restrict__ part2) {
     constexpr int LL = LM > 0 ? LM : 1;
-    constexpr int NV2 = (1 + LM) * B;
+    constexpr int NV1 = (1 + 2 * LM) * B, NV2 = (1 + LM) * B;
     __shared__ double lds[LZ_PUT_LDS];
+    __shared__ double sm[DIRECT ? NV1 : 1];
     const int b = threadIdx.x % B;
+    const double* S = DIRECT ? sm : a.st.sums;
+    if constexpr (DIRECT) {
+        const int nq = LM > 0 && a.st.so[0] == 1 ? 1 + 2 * LM : 1;  // sums of this step
+        const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+        for (int q = 0; q < nq; ++q) {
+            const int rows = q == 0 ? nk1 : nso;
+            double s = 0.0;
+#pragma unroll 4
+            for (int w = threadIdx.x / B; w < rows; w += LZ_WG / B) s += a.st.part[static_cast<size_t>(w) * NV1 + q * B + b];
+#pragma unroll
+            for (int o = B; o < 64; o <<= 1) s += __shfl_xor(s, o, 64);
+            if (lane < B) lds[wid * B + lane] = s;
+            __syncthreads();
+            if (threadIdx.x < B) {
+                double t = 0.0;
+                for (int w = 0; w < LZ_WG / 64; ++w) t += lds[w * B + threadIdx.x];
+                sm[q * B + threadIdx.x] = t;
+                if (blockIdx.x == 0) a.st.sums[q * B + threadIdx.x] = t;
+            }
+            __syncthreads();
+        }
+    }
     const int j = a.st.step[b];
     XT* vj = a.Xc;
     XT* vn = a.V + static_cast<int64_t>(j + 1) * a.vs;
     const bool act = a.st.active[b] != 0 && j < a.maxit;
     const double sj = a.st.scale[j * B + b];
-    const double al = a.st.sums[b], sg = lz_sigma<B>(a.st, b, j);
+    const double al = S[b], sg = lz_sigma<B>(a.st, b, j);
     const int mode = a.st.so[0];
     const int nl = (act && LM > 0 && mode != 0) ? min(a.st.nlock[b], LM) : 0;
     if (blockIdx.x == 0 && threadIdx.x < B && act) a.st.alpha[j * B + b] = al;
@@ -395,9 +423,9 @@ __global__ void __launch_bounds__(LZ_WG) __attribute__((amdgpu_waves_per_eu(LM =
             const int nll = (aa && mode != 0) ? min(a.st.nlock[bb], LM) : 0;
             double c = 0.0;
             if (l < nll) {
-                const double all = a.st.sums[bb];
+                const double all = S[bb];
                 if (mode == 1) {
-                    c = a.st.sums[(1 + l) * B + bb] - all * a.st.sums[(1 + LM + l) * B + bb];
+                    c = S[(1 + l) * B + bb] - all * S[(1 + LM + l) * B + bb];
                 } else {
                     const double bj = jj > 0 ? a.st.beta[jj * B + bb] : 0.0;
                     c = (a.st.ltheta[l * B + bb] - all) * a.st.dso[l * B + bb] - bj * a.st.dso[(LZ_LMAX + l) * B + bb];
@@ -478,10 +506,10 @@ __global__ void __launch_bounds__(LZ_WG) __attribute__((amdgpu_waves_per_eu(LM =
         }
     }
     if (LM > 0 && mode != 0) {  // uniform
-        lz_block_put_multi<B, 1 + LM>(acc, lds, a.st.part, NV2);
+        lz_block_put_multi<B, 1 + LM>(acc, lds, part2, NV2);
     } else {
         double a0[1] = {acc[0]};
-        lz_block_put_multi<B, 1>(a0, lds, a.st.part, NV2);
+        lz_block_put_multi<B, 1>(a0, lds, part2, NV2);
     }
 }
 
@@ -858,18 +886,31 @@ __global__ void __launch_bounds__(LZ_RED_WG) k_lz_reduce(const double* __restric
 // step's orthogonalisation flag.  K2's partial sums are first reduced by k_lz_reduce_wide (one workgroup per
 // value, fixed order) into `pre`; this one workgroup stages them in LDS, then updates the locked-vector
 // quantities with a thread per (vector, lane), then each lane's beta and step counter with a thread per lane
-// (the step counters are read by all of phase 2a before any is written).
+// (the step counters are read by all of phase 2a before any is written).  nwg > 0: it adds up those nwg rows of
+// partial sums at `pre` itself, a wave per value.
 constexpr int LZ_BETA_MAXV = (1 + LZ_LMAX) * 64;
 
 template <int B>
 __global__ void __launch_bounds__(LZ_RED_WG) k_lz_beta(LzState st, const double* __restrict__ pre, int nv, int maxit,
-                                                       double eps, int so_always) {
+                                                       double eps, int so_always, int nwg) {
     __shared__ double sums[LZ_BETA_MAXV];
     __shared__ int want;
     const int so_cur = st.so[0], so_prev = st.so[1];
     const int nvv = so_cur ? nv : B;
     if (threadIdx.x == 0) want = 0;
-    for (int v = threadIdx.x; v < nvv; v += LZ_RED_WG) sums[v] = pre[v];
+    if (nwg > 0) {
+        const int lane = threadIdx.x & 63;
+        for (int v = threadIdx.x >> 6; v < nvv; v += LZ_RED_WG / 64) {
+            double s = 0.0;
+#pragma unroll 4
+            for (int w = lane; w < nwg; w += 64) s += pre[static_cast<size_t>(w) * nv + v];
+#pragma unroll
+            for (int o = 32; o >= 1; o >>= 1) s += __shfl_xor(s, o, 64);
+            if (lane == 0) sums[v] = s;
+        }
+    } else {
+        for (int v = threadIdx.x; v < nvv; v += LZ_RED_WG) sums[v] = pre[v];
+    }
     __syncthreads();
     // phase 2a: one thread per (locked vector l, lane b), all in parallel
     for (int q = threadIdx.x; q < LZ_LMAX * B; q += LZ_RED_WG) {
@@ -2908,31 +2949,52 @@ class LzEngine final : public LzEngineBase {
             hipLaunchKernelGGL((k_lz_fr_beta<B>), dim3(1), dim3(LZ_RED_WG), 0, s, a, frs, gu, sums2.p, c);
         }
     }
+    void launch_k2(int LM, bool direct, double* part2) {
+#define K2(LL, DD) hipLaunchKernelGGL((k_lz_b<XT, B, LL, DD>), dim3(grid_k2), dim3(LZ_WG), 0, s, a, grid_k1, grid_so, part2)
+        if constexpr (B <= LZ_DIRECT_B) {
+            if (direct) {
+                if (LM == 0) K2(0, true);
+                else if (LM == 4) K2(4, true);
+                else if (LM == 8) K2(8, true);
+                else K2(16, true);
+                return;
+            }
+        }
+        if (LM == 0) K2(0, false);
+        else if (LM == 4) K2(4, false);
+        else if (LM == 8) K2(8, false);
+        else K2(16, false);
+#undef K2
+    }
     void step(int LM) {
         if (fullre) {
             step_fullre();
             return;
         }
         launch_k1(LM);
-        {
+        // Partial sums that are few are added up by the kernel that uses them, K1's by every workgroup of K2, K2's by the
+        // closing workgroup: two launches of five less (one lane: D = 24,310 14.0 -> 12.8 ms, 43,758 14.2 -> 13.4,
+        // 167,960 21.5 -> 21.1; eight mixed lanes of D = 92,378, 2,900 values of alpha, lost: 12.7 -> 13.3).  The lines
+        // lie at sizes alone, whatever the lanes' locked sets, so that a lane's sums are the same alone and in a mix.
+        const int nv = (1 + 2 * LM) * B, nv2 = (1 + LM) * B;
+        const size_t rows1 = std::max(grid_k1, grid_so), room = rows1 * (1 + 2 * LZ_LMAX) + static_cast<size_t>(grid_k2) * (1 + LZ_LMAX);
+        const bool direct = B <= LZ_DIRECT_B && grid_k1 * B <= 2048 && room * B <= part.n, direct2 = grid_k2 * B <= 1024;
+        double* part2 = direct ? part.p + rows1 * nv : part.p;  // K2 reads K1's partials while it writes its own
+        if (!direct) {
             KTimer kt(ctx, "lanczos_reduce", s);
-            const int nv = (1 + 2 * LM) * B;
             hipLaunchKernelGGL((k_lz_reduce_wide<B>), dim3(nv), dim3(LZ_RED_WG), 0, s, st, part.p, grid_k1, grid_so, nv, B, 0, st.sums);
         }
         {
             KTimer kt(ctx, "lanczos_update", s);
-            if (LM == 0) hipLaunchKernelGGL((k_lz_b<XT, B, 0>), dim3(grid_k2), dim3(LZ_WG), 0, s, a);
-            else if (LM == 4) hipLaunchKernelGGL((k_lz_b<XT, B, 4>), dim3(grid_k2), dim3(LZ_WG), 0, s, a);
-            else if (LM == 8) hipLaunchKernelGGL((k_lz_b<XT, B, 8>), dim3(grid_k2), dim3(LZ_WG), 0, s, a);
-            else hipLaunchKernelGGL((k_lz_b<XT, B, 16>), dim3(grid_k2), dim3(LZ_WG), 0, s, a);
+            launch_k2(LM, direct, part2);
         }
         {
             KTimer kt(ctx, "lanczos_reduce", s);
-            const int nv2 = (1 + LM) * B;
-            hipLaunchKernelGGL((k_lz_reduce_wide<B>), dim3(nv2), dim3(LZ_RED_WG), 0, s, st, part.p, grid_k2, grid_k2, nv2, B, 1,
-                               sums2.p);
-            hipLaunchKernelGGL((k_lz_beta<B>), dim3(1), dim3(LZ_RED_WG), 0, s, st, sums2.p, nv2, cap, eps_store,
-                               lz_so_always());
+            if (!direct2)
+                hipLaunchKernelGGL((k_lz_reduce_wide<B>), dim3(nv2), dim3(LZ_RED_WG), 0, s, st, part2, grid_k2, grid_k2, nv2, B, 1,
+                                   sums2.p);
+            hipLaunchKernelGGL((k_lz_beta<B>), dim3(1), dim3(LZ_RED_WG), 0, s, st, direct2 ? part2 : sums2.p, nv2, cap, eps_store,
+                               lz_so_always(), direct2 ? grid_k2 : 0);
         }
     }
     // Scratch of the finish, the deflations and the locks: a grow-only slot of the context workspace when the
