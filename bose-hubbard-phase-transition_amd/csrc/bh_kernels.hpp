@@ -42,53 +42,6 @@ __device__ __forceinline__ double bh_group_sum(double v) {
     return v;
 }
 
-// Sums NV values per vector b over the workgroup.  Each lane contributes v[0..NV-1] for its
-// b = lane % B.  On return, out[q * B + b] (LDS, NV*B doubles) holds the workgroup totals; all lanes
-// must call it.  scratch: (BH_WG/64) * B * NV doubles of LDS.
-template <int B, int NV>
-__device__ __forceinline__ void bh_block_sum_b(double (&v)[NV], double* scratch, double* out) {
-    const int lane = threadIdx.x & 63;
-    const int wid = threadIdx.x >> 6;
-#pragma unroll
-    for (int q = 0; q < NV; ++q) {
-        double t = v[q];
-#pragma unroll
-        for (int o = B; o < 64; o <<= 1) t += __shfl_xor(t, o, 64);
-        if (lane < B) scratch[(wid * NV + q) * B + lane] = t;
-    }
-    __syncthreads();
-    for (int i = threadIdx.x; i < NV * B; i += BH_WG) {
-        const int q = i / B, b = i % B;
-        double t = 0.0;
-        for (int w = 0; w < BH_WG / 64; ++w) t += scratch[(w * NV + q) * B + b];
-        out[i] = t;
-    }
-    __syncthreads();
-}
-
-// true in exactly one workgroup: the last one to arrive.  Partials written before the call by any
-// workgroup are visible to the last one after it returns.  The counter is reset by the caller.
-__device__ __forceinline__ bool bh_last_block(unsigned* counter) {
-    __shared__ int amlast;
-    __threadfence();
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        const unsigned prev = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
-        amlast = (prev == gridDim.x - 1) ? 1 : 0;
-    }
-    __syncthreads();
-    if (amlast) __threadfence();
-    return amlast != 0;
-}
-
-__device__ __forceinline__ double bh_coherent_load(const double* p) {
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-__device__ __forceinline__ void bh_reset_counter(unsigned* counter) {
-    __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
 // Row tile of a workgroup with XCD-aware placement.  Workgroups are dispatched round-robin over the
 // 8 XCDs of the chip (workgroup w runs on XCD w % 8); tile ids are renumbered so that each XCD walks
 // one contiguous eighth of the rows, keeping the x gathers of neighbouring rows in one L2.
