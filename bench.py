@@ -102,6 +102,14 @@ def run_cpu_child(mode, args, cap_s, threads, setup_cap_s=600.0):
     return recs, elapsed
 
 
+def ref_solver(args):
+    """Whether the reference's CPU solver is to be timed beside the device: not with --no-cpu, and not where
+    oracle/_ref has not been built (it needs the reference's sources); its figures are then null."""
+    import oracle as O
+
+    return not args.no_cpu and O.ref_available()
+
+
 def cpu_child(mode, argv):
     """Child side of run_cpu_child: builds the sector(s) with the oracle (host CSR in the reference's basis
     order), then runs the reference's own solver, printing one JSON record per finished solve."""
@@ -508,7 +516,7 @@ def main():
         ctx = bhx.Context(0)
         log("device:", bhx.device_name(0))
         serve = serving(ctx, args.serve, 200.0, args.serve_sustained)
-        if not args.no_cpu:
+        if ref_solver(args):
             serve["cpu_reference"] = serving_cpu()
         print(json.dumps({"serving": serve}))
         ctx.close()
@@ -644,7 +652,7 @@ def main():
         sweep = {"s": tsw, "solves": 3 * Jsw.size, "solves_per_s": 3 * Jsw.size / tsw, "width": rsw["width"].tolist(),
                  "fp64_reruns": int(rsw["used_fp64"].sum()), "all_ok": bool(np.all(rsw["status"] == 0)),
                  "rerun_causes": rerun_causes(ctx, Jsw, rsw["width"].tolist())}
-        if not args.no_cpu:
+        if ref_solver(args):
             sweep["cpu_reference"] = sweep_cpu(Jsw)
         log("sweep chain m=10 n=9/10/11:", json.dumps(sweep))
 
@@ -656,12 +664,12 @@ def main():
     serve = None
     if args.serve > 0 and not args.quick:
         serve = serving(ctx, args.serve, 200.0, args.serve_sustained)
-        if not args.no_cpu:
+        if ref_solver(args):
             serve["cpu_reference"] = serving_cpu()
         log("serving:", json.dumps(serve))
 
     cpu = None
-    if not args.no_cpu and not args.quick:
+    if not args.quick and ref_solver(args):
         cpu = cpu_baseline(Js, k)
         log("cpu baseline:", json.dumps(cpu))
 
