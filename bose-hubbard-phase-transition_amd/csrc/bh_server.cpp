@@ -12,6 +12,7 @@
 #include <condition_variable>
 #include <cstring>
 #include <deque>
+#include <iterator>
 #include <list>
 #include <map>
 #include <memory>
@@ -52,6 +53,7 @@ struct Sector {
     size_t ham_bytes = 0, eng_bytes[2] = {0, 0};
     bool never_fits = false;
     bool inflight[2] = {false, false};       // a chunk of the engine's steps is on its stream
+    bool evicted = false;                    // given up whole; leaves the map before the next pass (see worker_loop)
 };
 
 }  // namespace
@@ -136,7 +138,9 @@ void release_engine(bh_server* S, Sector& sc, int p) {
 // Frees memory until `need` more bytes fit: first idle engines (no busy lane) with nothing queued for them,
 // any sector's, least recently used first (an engine is rebuilt on demand; without this step two sectors
 // whose FP64 reruns wait for memory while each holds an idle mixed engine would wait for each other
-// forever), then idle sectors (no queue, no busy lane) whole.  `keep` / `keep_p` name the engine being made.
+// forever), then idle sectors (no queue, no busy lane) whole: their memory at once, their place in the map
+// once the pass over the sectors, which holds pointers to them, has ended.  `keep` / `keep_p` name the engine being
+// made.
 void evict_for(bh_server* S, size_t need, Sector* keep, int keep_p = -1) {
     const size_t budget = S->opts.hbm_budget;
     while (server_used(S) + need > budget) {
@@ -162,7 +166,7 @@ void evict_for(bh_server* S, size_t need, Sector* keep, int keep_p = -1) {
         Sector* victim = nullptr;
         for (auto& kv : S->sectors) {
             Sector* sc = kv.second.get();
-            if (sc == keep || !sc->queue[0].empty() || !sc->queue[1].empty()) continue;
+            if (sc == keep || sc->evicted || !sc->queue[0].empty() || !sc->queue[1].empty()) continue;
             bool busy = false;
             for (int p = 0; p < 2; ++p)
                 for (char c : sc->lane_busy[p]) busy |= c != 0;
@@ -173,7 +177,10 @@ void evict_for(bh_server* S, size_t need, Sector* keep, int keep_p = -1) {
         for (int p = 0; p < 2; ++p) release_engine(S, *victim, p);
         if (victim->ham) bh_ham_destroy(victim->ham);
         if (victim->basis) bh_basis_destroy(victim->basis);
-        S->sectors.erase(victim->key);
+        victim->ham = nullptr;
+        victim->basis = nullptr;
+        victim->ham_bytes = 0;
+        victim->evicted = true;
     }
     // Still short and no lane anywhere busy (nothing would ever free memory): the other sectors' CSRs are
     // released too, their queues kept (a sector builds its CSR again when it is served), so that the sector
@@ -414,6 +421,7 @@ bool advance(bh_server* S, Sector& sc, int p) {
 void worker_loop(bh_server* S) {
     (void)hipSetDevice(S->ctx->device);
     for (;;) {
+        for (auto it = S->sectors.begin(); it != S->sectors.end();) it = it->second->evicted ? S->sectors.erase(it) : std::next(it);
         {
             std::unique_lock<std::mutex> lk(S->mu);
             bool have_work = !S->inbox.empty();
@@ -436,7 +444,7 @@ void worker_loop(bh_server* S) {
             }
         }
         bool progressed = false;
-        std::vector<Sector*> small;
+        std::vector<Sector*> small;  // valid for the whole pass: a sector evicted in it stays in the map, empty
         for (auto& kv : S->sectors) {
             Sector& sc = *kv.second;
             if (sc.ham && sc.ham->D <= SRV_SMALL_D) {
