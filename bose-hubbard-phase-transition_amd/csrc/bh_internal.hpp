@@ -33,7 +33,7 @@ struct bh_ctx {
     void* ws[NWS] = {};
     size_t ws_bytes[NWS] = {};
     // memory kept between calls, within the budget together with `used` and given up where that has no room: one freed block
-    // for the next allocation of about its size (bh_dev_free) and the builders' scratch (BhScratch)
+    // for the next allocation of its size (bh_dev_free) and the builders' scratch (BhScratch)
     void* spare = nullptr;
     size_t spare_bytes = 0;
     void* scratch = nullptr;
@@ -72,9 +72,9 @@ int bh_set_error(const bh_ctx* ctx, int code, const std::string& msg);
 
 // budgeted device allocation (bytes counted against ctx->budget).  hipFree of a block from 32 MB up takes 0.22 ms (80 MB; 32 MB
 // and below 7 us), most of what building and dropping a sector costs beside its kernels, so the last such block
-// freed, up to BH_SPARE_MAX bytes, waits for the next allocation it fits (at most half as large again).  It is given up
-// when the budget or the device has no room beside it, and at the end of the context.  The device is
-// synchronised before a block is kept, as hipFree does.
+// freed, up to BH_SPARE_MAX bytes, waits for the next allocation of the same size (a larger block handed out for a smaller
+// request would be counted, and later kept, as the smaller one).  It is given up when the budget or the device has no
+// room beside it, and at the end of the context.  The device is synchronised before a block is kept, as hipFree does.
 constexpr size_t BH_SPARE_MIN = size_t(32) << 20, BH_SPARE_MAX = size_t(256) << 20;
 int bh_dev_alloc(bh_ctx* ctx, void** p, size_t bytes);
 void bh_dev_free(bh_ctx* ctx, void* p, size_t bytes);

@@ -59,7 +59,7 @@ BhScratch::~BhScratch() {
 
 int bh_dev_alloc(bh_ctx* ctx, void** p, size_t bytes) {
     *p = nullptr;
-    if (ctx->spare && ctx->spare_bytes >= bytes && ctx->spare_bytes - bytes <= bytes / 2 && ctx->used + ctx->spare_bytes + ctx->scratch_bytes <= ctx->budget) {
+    if (ctx->spare && ctx->spare_bytes == bytes && ctx->used + bytes + ctx->scratch_bytes <= ctx->budget) {
         *p = ctx->spare;
         ctx->spare = nullptr;
         ctx->spare_bytes = 0;

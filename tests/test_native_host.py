@@ -36,3 +36,9 @@ def test_server_gives_up_idle_sectors(server):
     """small sectors under a budget that holds one or two of them: an idle one is given up whole while a pass over the small
     sectors is under way"""
     run(server, "evict")
+
+
+def test_context_counts_what_it_holds(tmp_path):
+    """the blocks and scratch a context keeps between calls: counted at their size, within the budget, given up for an
+    allocation that needs their room"""
+    run(build(str(tmp_path / "memory"), os.path.join(CSRC, "bh_runtime.hip"), os.path.join(NATIVE, "memory_host.cpp")))
