@@ -249,8 +249,7 @@ int ensure_engine(bh_server* S, Sector& sc, int p) {
     // the FP64 engine serves the reruns of rejected mixed solves
     const bh_lanczos_opts lo = p == 0 ? S->opts.lanczos : bh_fallback_opts(S->opts.lanczos);
     const int L = lanes_wanted(S, sc, p);
-    const size_t need = bh_engine_bytes(sc.ham->D, prec, L, lo) +
-                        (prec == BH_PREC_FP64 ? static_cast<size_t>(sc.ham->nnz) * 12 : 0);
+    const size_t need = bh_engine_bytes(sc.ham->D, prec, L, lo);
     evict_for(S, need, &sc, p);
     if (server_used(S) + need > S->opts.hbm_budget) {
         if (need + sc.ham_bytes > S->opts.hbm_budget) sc.never_fits = true;

@@ -183,6 +183,13 @@ int main(int argc, char** argv) {
         stub::check(hams_built > 3, "no sector was given up");
         stub::check(bh_server_destroy(S) == BH_OK, "destroy");
         stub::check(stub::live.empty(), "streams or handles left behind");
+    } else if (what == "rerun") {
+        // a rejected mixed solve under a budget with room for the matrix (3,500 bytes) and two engines, and little more
+        accept_mixed = fullre = false;
+        bh_server* S = server(6000);
+        serve(S, 4, 4, 0.5, BH_OK);
+        stub::check(accept_mixed, "no rerun");
+        stub::check(bh_server_destroy(S) == BH_OK, "destroy");
     } else {
         stub::fail("unknown scenario");
     }

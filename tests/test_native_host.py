@@ -38,6 +38,11 @@ def test_server_gives_up_idle_sectors(server):
     run(server, "evict")
 
 
+def test_server_admits_a_rerun_that_fits(server):
+    """the FP64 engine of a rerun needs its own bytes beside the matrix, and no second matrix"""
+    run(server, "rerun")
+
+
 def test_context_counts_what_it_holds(tmp_path):
     """the blocks and scratch a context keeps between calls: counted at their size, within the budget, given up for an
     allocation that needs their room"""
