@@ -74,7 +74,7 @@ int bh_set_error(const bh_ctx* ctx, int code, const std::string& msg);
 // and below 7 us), most of what building and dropping a sector costs beside its kernels, so the last such block
 // freed, up to BH_SPARE_MAX bytes, waits for the next allocation of the same size (a larger block handed out for a smaller
 // request would be counted, and later kept, as the smaller one).  It is given up when the budget or the device has no
-// room beside it, and at the end of the context.  The device is synchronised before a block is kept, as hipFree does.
+// room beside it, and at the end of the context.  A block is kept once the device is idle, as hipFree would leave it.
 constexpr size_t BH_SPARE_MIN = size_t(32) << 20, BH_SPARE_MAX = size_t(256) << 20;
 int bh_dev_alloc(bh_ctx* ctx, void** p, size_t bytes);
 void bh_dev_free(bh_ctx* ctx, void* p, size_t bytes);

@@ -90,10 +90,19 @@ int bh_dev_alloc(bh_ctx* ctx, void** p, size_t bytes) {
     return BH_OK;
 }
 
+// Waits for the device as hipFree of a block does, by freeing a small one (1.5 us on an idle device): hipDeviceSynchronize
+// would end every stream capture under way, hipFree only those that forbid it to the calling thread.
+static bool wait_as_free() {
+    void* q = nullptr;
+    if (hipMalloc(&q, 256) == hipSuccess) return hipFree(q) == hipSuccess;
+    (void)hipGetLastError();
+    return false;
+}
+
 void bh_dev_free(bh_ctx* ctx, void* p, size_t bytes) {
     if (!p) return;
     const auto t0 = std::chrono::steady_clock::now();
-    if (bytes >= BH_SPARE_MIN && bytes <= BH_SPARE_MAX && hipDeviceSynchronize() == hipSuccess) {
+    if (bytes >= BH_SPARE_MIN && bytes <= BH_SPARE_MAX && wait_as_free()) {
         spare_release(ctx);
         ctx->spare = p;
         ctx->spare_bytes = bytes;

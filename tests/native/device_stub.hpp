@@ -57,7 +57,7 @@ hipError_t hipMemGetInfo(size_t* f, size_t* t) {
 }
 const char* hipGetErrorString(hipError_t) { return "stub"; }
 hipError_t hipGetLastError() { return hipSuccess; }
-hipError_t hipDeviceSynchronize() { return hipSuccess; }
+hipError_t hipDeviceSynchronize() { stub::fail("hipDeviceSynchronize ends the captures of other threads"); }
 hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) {
     *s = reinterpret_cast<hipStream_t>(std::malloc(1));
     stub::live.insert(*s);
