@@ -315,7 +315,7 @@ __global__ void __launch_bounds__(256) k_spdm(int64_t D, int m, int n, const uin
             double v[MAXM];
 #pragma unroll
             for (int j = 0; j < MAXM; ++j)
-                if (j < m && j > i0 + ii) {  // uniform; a source without a boson reads this state again, and adds zero
+                if (j < m && j > i0 + ii) {  // uniform; a source without a boson reads this state again, and adds nothing
                     const uint32_t t = s.get(j) >= 1 ? static_cast<uint32_t>(r) + di[ii] - dn[j] : static_cast<uint32_t>(r);
                     v[j] = phi[t];
                 }
@@ -323,7 +323,10 @@ __global__ void __launch_bounds__(256) k_spdm(int64_t D, int m, int n, const uin
             for (int j = 0; j < MAXM; ++j)
                 if (j < m && j > i0 + ii) {
                     const int c = (ni[ii] + 1) * s.get(j);
-                    acc[ii][j] += pq * v[j] * (nsq ? sq[c] : std::sqrt(static_cast<double>(c)));
+                    // no boson on j: the factor is 0, and the product of the amplitudes must not be infinite or NaN
+                    // (its low word alone is finite)
+                    const double pv = pq * v[j], f = __hiloint2double(s.get(j) >= 1 ? __double2hiint(pv) : 0, __double2loint(pv));
+                    acc[ii][j] += f * (nsq ? sq[c] : std::sqrt(static_cast<double>(c)));
                 }
         }
     }
