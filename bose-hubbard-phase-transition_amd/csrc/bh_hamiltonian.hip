@@ -745,14 +745,29 @@ int bh_spdm(bh_ctx* ctx, const bh_basis* b, const double* phi, double* rho) {
     const size_t lds_bytes = static_cast<size_t>(nsq) * 8 + static_cast<size_t>(gsize) * 4;
     const int nb = static_cast<int>(std::min<int64_t>((D + 255) / 256, 768));
     const bool lex = b->order == BH_ORDER_LEX;
+    const size_t vb = BhScratch::size(D * 8), sums = BhScratch::size(static_cast<size_t>(m) * m * nb * 8) + BhScratch::size(static_cast<size_t>(m) * m * 8);
     BhScratch sc;
-    BH_TRY(sc.open(ctx, BhScratch::size(D * 8) * (lex ? 1 : 2) + BhScratch::size(static_cast<size_t>(m) * m * nb * 8) +
-                            BhScratch::size(static_cast<size_t>(m) * m * 8)));
+    int rc = sc.open(ctx, vb * (lex ? 1 : 2) + sums);
+    // where there is no room for a second vector the host brings phi into lexicographic order
+    const bool host = rc != BH_OK && !lex;
+    if (host) {
+        (void)hipGetLastError();
+        rc = sc.open(ctx, vb + sums);
+    }
+    if (rc != BH_OK) return rc;
     double* dphi = sc.take<double>(D);
     double* part = sc.take<double>(static_cast<size_t>(m) * m * nb);
     double* out = sc.take<double>(static_cast<size_t>(m) * m);
-    BH_HIP(ctx, hipMemcpyAsync(dphi, phi, static_cast<size_t>(D) * 8, hipMemcpyHostToDevice, s));
-    if (!lex) {
+    std::vector<double> hphi;
+    if (host) {
+        std::vector<int32_t> pol(static_cast<size_t>(D));
+        hphi.resize(static_cast<size_t>(D));
+        BH_HIP(ctx, hipMemcpyAsync(pol.data(), b->pos_of_lex, pol.size() * sizeof(int32_t), hipMemcpyDeviceToHost, s));
+        BH_HIP(ctx, hipStreamSynchronize(s));
+        for (int64_t r = 0; r < D; ++r) hphi[r] = phi[pol[r]];
+    }
+    BH_HIP(ctx, hipMemcpyAsync(dphi, host ? hphi.data() : phi, static_cast<size_t>(D) * 8, hipMemcpyHostToDevice, s));
+    if (!lex && !host) {
         double* pl = sc.take<double>(D);
         hipLaunchKernelGGL(k_gather_f64, dim3(static_cast<unsigned>((D + 255) / 256)), dim3(256), 0, s, D, b->pos_of_lex, dphi, pl);
         dphi = pl;
