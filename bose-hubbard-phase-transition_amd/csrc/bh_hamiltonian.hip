@@ -542,7 +542,7 @@ int bh_hamiltonian_build(bh_ctx* ctx, const bh_basis* b, const int* nbr_off, con
 
     // every directed bond (i, j) contributes an entry per state with a boson on j
     const int64_t per_bond = n >= 1 ? bh_binom_host(m + n - 2, n - 1) : 0;
-    if (per_bond < 0 || per_bond > INT32_MAX || static_cast<int64_t>(E) * per_bond > INT32_MAX)
+    if (per_bond < 0 || per_bond > BH_NNZ_MAX || static_cast<int64_t>(E) * per_bond > BH_NNZ_MAX)
         return bh_set_error(ctx, BH_ERANGE, "hamiltonian: number of entries exceeds the int32 index range");
     const int64_t nnz = E * per_bond;
     SiteDeg deg{};

@@ -231,6 +231,10 @@ int bh_engine_env();  // BHX_ENGINE (-1 when unset)
 
 constexpr int BH_MAX_SITES = 32;
 constexpr int BH_WORDS_PAD = 4;  // words past the last entry that a 16-byte load may read (their values are not used)
+// entries of a Hamiltonian at most: the kernels' 32-bit word indexes run up to a tile (BH_TILE_WORDS + 1,024 words) or an unrolled
+// step past the last one.  No sector has a number of entries between this and the int32 limit (the largest below
+// it is 18 sites, 12 bosons, 100 directed bonds: 2,147,418,000), so the room refuses nothing.
+constexpr int64_t BH_NNZ_MAX = INT32_MAX - 8192;
 constexpr int BH_STAGE_PRODUCTS_HOST = 2048;  // must equal BH_STAGE_PRODUCTS of the row-block engine
 extern const int bh_primes[BH_MAX_SITES];
 

@@ -1,6 +1,8 @@
 """Host code of the library on a stand-in device (tests/native): compiled for the host alone and run here, where a use of
 released memory or of a released handle ends the program with a message instead of going on."""
+import math
 import os
+import re
 import subprocess
 
 import pytest
@@ -47,3 +49,24 @@ def test_context_counts_what_it_holds(tmp_path):
     """the blocks and scratch a context keeps between calls: counted at their size, within the budget, given up for an
     allocation that needs their room"""
     run(build(str(tmp_path / "memory"), os.path.join(CSRC, "bh_runtime.hip"), os.path.join(NATIVE, "memory_host.cpp")))
+
+
+def test_no_sector_between_the_entry_limits():
+    """the room that the kernels' index arithmetic needs below the int32 limit refuses no sector: none that the word format
+    takes (column and code in 32 bits, at most 12 of them the code) has a number of entries in it"""
+    src = open(os.path.join(CSRC, "bh_internal.hpp")).read()
+    room = int(re.search(r"BH_NNZ_MAX = INT32_MAX - (\d+);", src).group(1))
+    top, nearest = 2**31 - 1, 0
+    for m in range(2, 33):
+        for n in range(1, 256):
+            D = math.comb(m + n - 1, n)
+            code = max((n - q + 1) * q for q in range(1, n + 1))  # single bonds: the narrowest code
+            cb = code.bit_length()
+            if cb > 12 or (D - 1) >> (32 - cb):
+                continue
+            per_bond = math.comb(m + n - 2, n - 1)
+            for E in range(2, min(128, m * (m - 1)) + 1, 2):
+                if E * per_bond <= top:
+                    nearest = max(nearest, E * per_bond)
+    assert nearest == 2147418000 and nearest <= top - room
+    assert room >= 2048 + 1024 + 64
