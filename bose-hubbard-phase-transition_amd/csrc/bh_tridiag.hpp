@@ -9,20 +9,6 @@
 
 namespace bhtri {
 
-// number of eigenvalues of T strictly below x (negative pivots of the LDL^T of T - x I)
-inline int sturm_count(int n, const double* a, const double* b, double x, double tiny) {
-    int c = 0;
-    double q = a[0] - x;
-    if (q == 0.0) q = -tiny;
-    if (q < 0) ++c;
-    for (int t = 1; t < n; ++t) {
-        q = (a[t] - x) - b[t] * b[t] / q;
-        if (q == 0.0) q = -tiny;
-        if (q < 0) ++c;
-    }
-    return c;
-}
-
 inline void gershgorin(int n, const double* a, const double* b, double* lo, double* hi) {
     double l = a[0], h = a[0];
     for (int t = 0; t < n; ++t) {
@@ -34,22 +20,10 @@ inline void gershgorin(int n, const double* a, const double* b, double* lo, doub
     *hi = h;
 }
 
-// eigenvalue of index idx (0 = smallest), to about 2 eps |x|
-inline double bisect(int n, const double* a, const double* b, int idx, double lo, double hi) {
-    const double tiny = 1e-300 + 1e-18 * std::fmax(std::fabs(lo), std::fabs(hi));
-    for (int it = 0; it < 200; ++it) {
-        const double mid = 0.5 * (lo + hi);
-        if (mid <= lo || mid >= hi) break;
-        if (hi - lo <= 4.0e-16 * std::fmax(std::fabs(lo), std::fabs(hi))) break;
-        if (sturm_count(n, a, b, mid, tiny) > idx) hi = mid;
-        else lo = mid;
-    }
-    return 0.5 * (lo + hi);
-}
-
-// the p lowest eigenvalues, each the same sequence of midpoints and counts as bisect(i), eight of them side by side:
-// one Sturm recurrence is a chain of dependent divisions (about 22 cycles a row), eight independent ones keep the
-// divider busy (twelve values of a 150-row T: 0.6 -> 0.1 ms)
+// the p lowest eigenvalues of T, to about 2 eps |x|: bisection between lo0 and hi0, where the count of eigenvalues below x is
+// the number of negative pivots of the LDL^T of T - x I (a zero pivot counts as a tiny negative one).  One Sturm recurrence
+// is a chain of dependent divisions (about 22 cycles a row), so eight of them run side by side, each with its own
+// interval, and keep the divider busy (twelve values of a 150-row T: 0.6 -> 0.1 ms)
 inline void bisect_lowest(int n, const double* a, const double* b, int p, double lo0, double hi0, double* out) {
     constexpr int W = 8;
     const double tiny = 1e-300 + 1e-18 * std::fmax(std::fabs(lo0), std::fabs(hi0));
