@@ -261,12 +261,12 @@ def mean_field_leg(ctx, cpu_sample, n=1000, precision=5):
 PROFILE = os.path.join(ROOT, "profiles", "k1_lanczos_mixed_b16_chain12.txt")
 
 
-def traffic_from_profile():
-    """HBM bytes per K1 launch measured by rocprofv3 FETCH_SIZE / WRITE_SIZE passes on this workload (the
-    committed summary holds the command, the copy-kernel calibration and the figure); None without it."""
+def traffic_from_profile(B, tuned):
+    """HBM bytes per K1 launch measured by rocprofv3 FETCH_SIZE / WRITE_SIZE passes on this workload for the variant in use
+    (the committed summary holds the commands, the copy-kernel calibration and the figures); None for others."""
     try:
         for line in open(PROFILE):
-            if line.startswith("traffic_bytes_per_launch:"):
+            if B == 16 and tuned and line.startswith(f"traffic_bytes_per_launch[{tuned['variant']}]:"):
                 return float(line.split(":")[1])
     except OSError:
         pass
@@ -699,8 +699,8 @@ def main():
         "mean_field_1000x1000": mf,
         "serving": serve,
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                     "frac": achieved / HBM_PEAK_GBS, "traffic": traffic_from_profile()},
-        "k1": {"kernel": "k_lz_a_rl (fused Lanczos operator pass)", "launches": k1_count, "avg_us": k1_ms * 1e3,
+                     "frac": achieved / HBM_PEAK_GBS, "traffic": traffic_from_profile(B, k1_tuned)},
+        "k1": {"kernel": "k_lz_a_rl, k_lz_a_rlw (fused Lanczos operator pass)", "launches": k1_count, "avg_us": k1_ms * 1e3,
                "alg_bytes_per_launch": k1_bytes, "k2_avg_us": upd_total / max(upd_count, 1) * 1e3,
                "tuned": k1_tuned},
         "cpu_baseline": cpu,
